@@ -47,6 +47,12 @@ enum { SPECT_F32 = 0, SPECT_F64 = 1 };
  * (mu must still be non-NULL; it is not read). */
 enum { SPECT_ATT_FIELD = 0x100 };
 
+/* Flag OR-ed into the dtype argument of spect_forward and spect_backward: blur
+ * every plane with its own PSF, as the transposes and derivatives of those calls
+ * do, where a float32 call may otherwise blur a few combined images that
+ * represent the planes' PSFs to 2^-22. */
+enum { SPECT_PLANES = 0x200 };
+
 /* Padding modes of spect_smooth_axis (torch Conv1d padding_mode). */
 enum { SPECT_PAD_CIRCULAR = 0, SPECT_PAD_REPLICATE = 1, SPECT_PAD_ZEROS = 2 };
 
@@ -109,7 +115,8 @@ int spect_plan_dims(const spect_plan *p, int32_t *padded, int32_t *pad, int32_t 
 size_t spect_workspace_bytes(const spect_plan *p, int dtype, int n);
 
 /* The plane schedule an n-angle call runs with this plan, dtype and the
- * device current now (sched_rounds of spect_geom): *forward = 1 when the
+ * device current now (sched_rounds of spect_geom; a float32 call that blurs
+ * combined images, see SPECT_PLANES, runs no such schedule): *forward = 1 when the
  * forward projection (no attenuation, or the attenuation field) runs the
  * balanced schedule, 0 for uniform chunks; *field likewise for the back
  * projection's field kernel.  No counterpart in the reference: a diagnostic of

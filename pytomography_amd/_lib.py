@@ -17,6 +17,7 @@ LIB_PATH = os.path.join(_HERE, "libspect_hip.so")
 
 SPECT_F32, SPECT_F64 = 0, 1
 ATT_FIELD = 0x100  # OR-ed into dtype: att_table is an attenuation field
+PLANES = 0x200  # OR-ed into dtype: blur every plane with its own PSF
 BP_REFERENCE, BP_ADJOINT = 0, 1
 PAD_CIRCULAR, PAD_REPLICATE, PAD_ZEROS = 0, 1, 2
 OUT_STORE, OUT_ADD, OUT_OSEM = 0, 1, 2

@@ -7,11 +7,14 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/spect_hip.h"
 #include "launch.hpp"
 #include "activity.hpp"
+#include "lowrank.hpp"
+#include "lowrank_launch.hpp"
 #include "tiers.hpp"
 
 #define SPECT_VERSION 2
@@ -40,6 +43,8 @@ struct spect_plan {
   int32_t *tier32 = nullptr, *tier64 = nullptr;  // [n_radii][P] blur tier per plane
   unsigned long long *act = nullptr;  // [A][ntiles][C] visited planes per forward block
   int2 *ranges = nullptr;             // [A][ntiles] visited plane range per (angle, tile)
+  LrTables lr{};                      // float32 combined images (nseg 0: not used)
+  void *lr_mem[7] = {};               // their device tables
 };
 
 namespace {
@@ -131,8 +136,46 @@ template <typename R> Geo<R> geo(const spect_plan *p) {
   return g;
 }
 
+// Device tables of the combined images (lowrank.hpp) from the taps of every
+// radius ([n_radii][P][2H+1], float64 when the plan has them: they are free of
+// the float32 rounding that the fit would otherwise reproduce).  Leaves
+// p->lr.nseg at 0 -- the planes are then blurred one by one -- when they do not
+// represent the PSF, or the object or one angle of the field reaches the
+// kernels' 32-bit offsets.
+template <typename T>
+int lowrank_build(spect_plan *p, const T *taps_r, const T *taps_z) {
+  const Geo<float> g = geo<float>(p);
+  const size_t limit = (size_t)1 << 32;
+  if ((size_t)p->N * p->N * p->Nz * 4 >= limit || (size_t)p->P * (g.je1 - g.je0) * p->Nz * 4 >= limit)
+    return SPECT_OK;
+  LrHostTables t;
+  if (!lowrank_tables<T>(taps_r, taps_z, p->n_radii, p->P, p->H, t)) return SPECT_OK;
+  int rc = SPECT_OK, k = 0;
+  auto up = [&](const auto &v) {
+    using E = std::remove_const_t<std::remove_pointer_t<decltype(v.data())>>;
+    E *d = nullptr;
+    if (!rc) rc = upload(&d, v.data(), v.size());
+    p->lr_mem[k++] = d;
+    return d;
+  };
+  static_assert(sizeof(LrHostTables::Img) == sizeof(int4), "image descriptors are int4 on the device");
+  LrTables lr{};
+  lr.nseg = t.nseg;
+  lr.nimg = t.nimg;
+  lr.quads = t.quads;
+  lr.seg_unit = up(t.seg_unit);
+  lr.seg_rows = up(t.seg_rows);
+  lr.count = up(t.count);
+  lr.img = reinterpret_cast<const int4 *>(up(t.img));
+  lr.taps = up(t.taps);
+  lr.cf = up(t.cf);
+  lr.cb = up(t.cb);
+  if (!rc) p->lr = lr;
+  return rc;
+}
+
 struct Ws {
-  size_t att_off, part_off, w_off, ratio_off, total;
+  size_t att_off, part_off, w_off, q_off, ratio_off, total;
 };
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -187,13 +230,18 @@ Ws ws_layout(const spect_plan *p, int dtype, int n) {
   const Geo<float> g = geo<float>(p);
   const size_t n_jext = g.je1 - g.je0;
   const size_t att = align256((size_t)n * p->C * n_jext * p->Nz * sizeof(double));
-  const size_t part = fwd_part_layout(p, dtype, n).total;
-  const size_t w = align256((size_t)n * p->P * n_jext * p->Nz * rs);
+  size_t part = fwd_part_layout(p, dtype, n).total;
+  size_t w = align256((size_t)n * p->P * n_jext * p->Nz * rs);
   const size_t ratio = align256((size_t)n * p->N * p->Nz * rs);
   Ws l;
   l.att_off = 0;
   l.part_off = att;
   l.w_off = att;  // forward partials are consumed before the field is written
+  l.q_off = att + w;
+  if (dtype == SPECT_F32 && p->lr.nseg > 0) {
+    part = std::max(part, lr_forward_bytes(p->lr, g, n));
+    w += lr_backward_bytes(p->lr, g, n);
+  }
   l.ratio_off = att + std::max(part, w);
   l.total = l.ratio_off + ratio;
   return l;
@@ -262,19 +310,43 @@ int att_rows(const spect_plan *p, const Geo<R> &g, const R *mu, const void *tabl
   return SPECT_OK;
 }
 
+// Whether a float32 call blurs combined images (lowrank.hpp): a PSF that they
+// represent, and the attenuation factors as a field or no attenuation (the
+// suffix table's march carries a state from plane to plane).
+bool lr_runs(const spect_plan *p, const float *attf, const float *mu) {
+  return p->lr.nseg > 0 && (attf || !mu);
+}
+
 // Forward projection with its scratch given explicitly: rows (FP64
 // attenuation rows, used only with mu and no table) and part (the chunk
-// partials).
+// partials, or the combined images; part_bytes of them).
 template <typename R>
 int forward_core(const spect_plan *p, const R *f, const R *mu, const void *table, bool field,
                  const int32_t *idx, int n, R *proj, const R *gm, const R *s, R *pred, R *ratio,
-                 R delta, double *rows, R *part, hipStream_t st, bool trb) {
+                 R delta, double *rows, R *part, size_t part_bytes, hipStream_t st, bool trb, bool planes) {
   const Geo<R> g = geo<R>(p);
   const double *att;
   bool global;
   const R *attf;
   int rc = att_rows<R>(p, g, mu, table, field, idx, n, rows, st, &att, &global, &attf);
   if (rc) return rc;
+  if constexpr (sizeof(R) == 4) {
+    if (!trb && !planes && lr_runs(p, attf, mu)) {
+      // as many angles per launch as the scratch holds images for (all of them
+      // in a caller's workspace; the angles are independent)
+      int k = n;
+      while (k > 1 && lr_forward_bytes(p->lr, g, k) > part_bytes) k = (k + 1) / 2;
+      if (lr_forward_bytes(p->lr, g, k) <= part_bytes) {
+        const size_t rows_n = (size_t)(g.jo1 - g.jo0) * g.Nz;
+        auto at = [&](auto *q, size_t a) { return q ? q + a * rows_n : q; };
+        for (int a = 0; a < n; a += k)
+          HIP_TRY(launch_lr_forward(g, tables<R>(p), p->lr, f, attf, idx + a, std::min(k, n - a), at(proj, a),
+                                    at(gm, a), at(s, a), at(pred, a), at(ratio, a), delta,
+                                    reinterpret_cast<unsigned char *>(part), part_bytes, st));
+        return SPECT_OK;
+      }
+    }
+  }
   const FwdPart pl = fwd_part_layout(p, sizeof(R) == 8 ? SPECT_F64 : SPECT_F32, n);
   if (!trb && (attf || !mu) && pl.sched_blocks > 0) {
     // the balanced schedule: every block carries the same number of planes
@@ -292,18 +364,18 @@ int forward_core(const spect_plan *p, const R *f, const R *mu, const void *table
 template <typename R>
 int forward_impl(const spect_plan *p, const R *f, const R *mu, const void *table, bool field,
                  const int32_t *idx, int n, R *proj, const R *gm, const R *s, R *pred, R *ratio,
-                 R delta, unsigned char *ws, hipStream_t st, bool trb = false) {
+                 R delta, unsigned char *ws, hipStream_t st, bool trb = false, bool planes = false) {
   const Ws l = ws_layout(p, sizeof(R) == 8 ? SPECT_F64 : SPECT_F32, n);
   return forward_core<R>(p, f, mu, table, field, idx, n, proj, gm, s, pred, ratio, delta,
                          reinterpret_cast<double *>(ws + l.att_off),
-                         reinterpret_cast<R *>(ws + l.part_off), st, trb);
+                         reinterpret_cast<R *>(ws + l.part_off), l.ratio_off - l.part_off, st, trb, planes);
 }
 
 template <typename R>
 int backward_impl(const spect_plan *p, int mode, int out_mode, const R *proj, const R *mu,
                   const void *table, bool field, const int32_t *idx, int n, R *out, const R *f,
                   const R *nrm, double delta, double floor_value, unsigned char *ws,
-                  hipStream_t st) {
+                  hipStream_t st, bool planes = false) {
   const Geo<R> g = geo<R>(p);
   const Ws l = ws_layout(p, sizeof(R) == 8 ? SPECT_F64 : SPECT_F32, n);
   const double *att;
@@ -323,6 +395,14 @@ int backward_impl(const spect_plan *p, int mode, int out_mode, const R *proj, co
     return SPECT_OK;
   }
   R *W = reinterpret_cast<R *>(ws + l.w_off);
+  if constexpr (sizeof(R) == 4) {
+    if (!planes && lr_runs(p, attf, mu) && lr_back_pays(g, n)) {
+      HIP_TRY(launch_lr_field(g, tables<R>(p), p->lr, proj, attf, idx, n, W, ws + l.q_off, l.ratio_off - l.q_off, st));
+      HIP_TRY(launch_bp_gather<R>(g, tables<R>(p), W, idx, n, mode, out_mode, out, f, nrm, R(delta),
+                                  R(floor_value), nullptr, nullptr, nullptr, st));
+      return SPECT_OK;
+    }
+  }
   const int fb = (attf || !mu) && p->rounds >= 0 ? std::max(1, p->rounds) * field_sched_blocks<R>(g)
                                                   : 0;
   if (sched_auto_ok(p, n, fb)) {
@@ -791,6 +871,9 @@ int spect_plan_create(const spect_geom *g, spect_plan **out) {
     if ((rc = upload(&p->taps_z32, z32.data(), z32.size()))) return cleanup(rc);
     auto t32v = tap_tiers<float>(r32.data(), z32.data(), rows, H, kTierEps32);
     if ((rc = upload(&p->tier32, t32v.data(), t32v.size()))) return cleanup(rc);
+    if (!p->has64) {
+      if ((rc = lowrank_build<float>(p, r32.data(), z32.data()))) return cleanup(rc);
+    }
     if (p->has64) {
       auto r64 = widen_taps<double>(g->taps_r64, rows, g->psf_kr, K, false);
       auto z64 = widen_taps<double>(g->psf_kz > 0 ? g->taps_z64 : nullptr, rows, g->psf_kz, K, true);
@@ -798,6 +881,7 @@ int spect_plan_create(const spect_geom *g, spect_plan **out) {
       if ((rc = upload(&p->taps_z64, z64.data(), z64.size()))) return cleanup(rc);
       auto t64v = tap_tiers<double>(r64.data(), z64.data(), rows, H, kTierEps64);
       if ((rc = upload(&p->tier64, t64v.data(), t64v.size()))) return cleanup(rc);
+      if ((rc = lowrank_build<double>(p, r64.data(), z64.data()))) return cleanup(rc);
     }
   }
   *out = p;
@@ -820,6 +904,7 @@ int spect_plan_destroy(spect_plan *p) {
   (void)hipFree(p->tier64);
   (void)hipFree(p->act);
   (void)hipFree(p->ranges);
+  for (void *m : p->lr_mem) (void)hipFree(m);
   delete p;
   return SPECT_OK;
 }
@@ -905,7 +990,8 @@ int spect_forward(const spect_plan *p, int dtype, const void *f, const void *mu,
                   const void *att_table, const int32_t *angle_idx, int n, void *proj,
                   void *workspace, size_t workspace_bytes, void *stream) {
   const bool field = (dtype & SPECT_ATT_FIELD) != 0;
-  dtype &= ~SPECT_ATT_FIELD;
+  const bool planes = (dtype & SPECT_PLANES) != 0;
+  dtype &= ~(SPECT_ATT_FIELD | SPECT_PLANES);
   if (int rc = check_call(p, dtype, n, workspace, workspace_bytes)) return rc;
   if (!f || !proj || !angle_idx) return fail(SPECT_E_ARG, "null array argument");
   if (int rc = check_arrays({f, mu, att_table, proj})) return rc;
@@ -913,7 +999,8 @@ int spect_forward(const spect_plan *p, int dtype, const void *f, const void *mu,
   auto *ws = reinterpret_cast<unsigned char *>(workspace);
   if (dtype == SPECT_F32)
     return forward_impl<float>(p, (const float *)f, (const float *)mu, att_table, field, angle_idx,
-                               n, (float *)proj, nullptr, nullptr, nullptr, nullptr, 0.f, ws, st);
+                               n, (float *)proj, nullptr, nullptr, nullptr, nullptr, 0.f, ws, st,
+                               false, planes);
   return forward_impl<double>(p, (const double *)f, (const double *)mu, att_table, field, angle_idx,
                               n, (double *)proj, nullptr, nullptr, nullptr, nullptr, 0.0, ws, st);
 }
@@ -991,10 +1078,12 @@ int spect_forward_noalloc(const spect_plan *p, int dtype, const void *f, const v
   if (dtype == SPECT_F32)
     return forward_core<float>(p, (const float *)f, (const float *)mu, att_table, field, angle_idx,
                                n, (float *)proj, nullptr, nullptr, nullptr, nullptr, 0.f, rows,
-                               reinterpret_cast<float *>(base + rows_b), st, false);
+                               reinterpret_cast<float *>(base + rows_b),
+                               SPECT_NOALLOC_SCRATCH_BYTES - rows_b, st, false, false);
   return forward_core<double>(p, (const double *)f, (const double *)mu, att_table, field, angle_idx,
                               n, (double *)proj, nullptr, nullptr, nullptr, nullptr, 0.0, rows,
-                              reinterpret_cast<double *>(base + rows_b), st, false);
+                              reinterpret_cast<double *>(base + rows_b),
+                              SPECT_NOALLOC_SCRATCH_BYTES - rows_b, st, false, false);
 }
 
 int spect_backward_transpose(const spect_plan *p, int dtype, const void *v, const void *mu,
@@ -1021,7 +1110,8 @@ int spect_backward(const spect_plan *p, int dtype, int mode, int out_mode, const
                    void *out, const void *f, const void *norm, double delta, double floor_value,
                    void *workspace, size_t workspace_bytes, void *stream) {
   const bool field = (dtype & SPECT_ATT_FIELD) != 0;
-  dtype &= ~SPECT_ATT_FIELD;
+  const bool planes = (dtype & SPECT_PLANES) != 0;
+  dtype &= ~(SPECT_ATT_FIELD | SPECT_PLANES);
   if (int rc = check_call(p, dtype, n, workspace, workspace_bytes)) return rc;
   if (!proj || !out || !angle_idx) return fail(SPECT_E_ARG, "null array argument");
   if (mode != SPECT_BP_REFERENCE && mode != SPECT_BP_ADJOINT) return fail(SPECT_E_ARG, "bad mode");
@@ -1033,7 +1123,7 @@ int spect_backward(const spect_plan *p, int dtype, int mode, int out_mode, const
   if (dtype == SPECT_F32)
     return backward_impl<float>(p, mode, out_mode, (const float *)proj, (const float *)mu,
                                 att_table, field, angle_idx, n, (float *)out, (const float *)f,
-                                (const float *)norm, delta, floor_value, ws, st);
+                                (const float *)norm, delta, floor_value, ws, st, planes);
   return backward_impl<double>(p, mode, out_mode, (const double *)proj, (const double *)mu,
                                att_table, field, angle_idx, n, (double *)out, (const double *)f,
                                (const double *)norm, delta, floor_value, ws, st);

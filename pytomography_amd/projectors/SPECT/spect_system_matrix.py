@@ -147,7 +147,9 @@ class SPECTSystemMatrix(SystemMatrix):
         return ws, ws.numel()
 
     def schedule(self, subset_idx: int | None = None, dtype: torch.dtype | None = None) -> dict:
-        """The plane schedule the fused kernels run for this subset's angles
+        """The plane schedule that kernels which blur every plane run for this
+        subset's angles (float32 calls with a PSF may blur combined images
+        instead, csrc/lowrank_launch.hpp, and then have none)
         (``spect_schedule_info``): ``{"forward": ..., "field": ...}`` with
         "balanced" (pieces of the visited planes over one round of resident
         blocks) or "uniform" (``chunk_planes``-plane chunks); "forward" is the
@@ -225,9 +227,10 @@ class SPECTSystemMatrix(SystemMatrix):
         return tab
 
     @staticmethod
-    def _code(dt, tab) -> int:
-        """dtype argument of the projection entry points for attenuation data ``tab``."""
-        code = _lib.dtype_code(dt)
+    def _code(dt, tab, planes=False) -> int:
+        """dtype argument of the projection entry points for attenuation data ``tab``;
+        ``planes``: as the transposes and derivatives run (_lib.PLANES)."""
+        code = _lib.dtype_code(dt) | (_lib.PLANES if planes else 0)
         return code | _lib.ATT_FIELD if tab is not None and tab.att_field else code
 
     @staticmethod
@@ -354,7 +357,7 @@ class SPECTSystemMatrix(SystemMatrix):
         self._require_fused("backward_transpose")
         return self._project(object, subset_idx, "spect_backward_transpose")
 
-    def _project(self, object: torch.Tensor, subset_idx, entry: str) -> torch.Tensor:
+    def _project(self, object: torch.Tensor, subset_idx, entry: str, planes: bool = False) -> torch.Tensor:
         device = pytomography_amd.device if object.device.type != "cuda" else object.device
         dt = self._compute_dtype(object)
         f = _lib.require_device_tensor(object.to(device), "object", dt)
@@ -367,14 +370,14 @@ class SPECTSystemMatrix(SystemMatrix):
         tab = self._att_table(device, dt)
         out = torch.empty((n, self._shape[1], self._shape[2]), dtype=dt, device=device)
         ws, nbytes = self._workspace(device, dt, n)
-        _lib.check(getattr(plan.lib, entry)(plan.handle, self._code(dt, tab), f.data_ptr(),
+        _lib.check(getattr(plan.lib, entry)(plan.handle, self._code(dt, tab, planes), f.data_ptr(),
                                             _lib.ptr(mu), _lib.ptr(tab), idx.data_ptr(), n,
                                             out.data_ptr(), ws.data_ptr(), nbytes,
                                             _lib.stream_ptr(device)))
         return out
 
     def _backward(self, proj, subset_idx, mode, out_mode=_lib.OUT_STORE, out=None, f=None,
-                  norm=None, floor_value=0.0):
+                  norm=None, floor_value=0.0, planes=False):
         device = pytomography_amd.device if proj.device.type != "cuda" else proj.device
         dt = self._compute_dtype(proj)
         p = _lib.require_device_tensor(proj.to(device), "proj", dt)
@@ -389,7 +392,7 @@ class SPECTSystemMatrix(SystemMatrix):
             out = torch.empty(self._shape, dtype=dt, device=device)
         ws, nbytes = self._workspace(device, dt, n)
         _lib.check(plan.lib.spect_backward(
-            plan.handle, self._code(dt, tab), mode, out_mode, p.data_ptr(), _lib.ptr(mu),
+            plan.handle, self._code(dt, tab, planes), mode, out_mode, p.data_ptr(), _lib.ptr(mu),
             _lib.ptr(tab), idx.data_ptr(), n, out.data_ptr(), _lib.ptr(f), _lib.ptr(norm),
             float(pytomography_amd.delta), float(floor_value), ws.data_ptr(), nbytes,
             _lib.stream_ptr(device)))
@@ -454,7 +457,7 @@ class SPECTSystemMatrix(SystemMatrix):
         n = idx.numel()
         out = torch.empty((n, self._shape[1], self._shape[2]), dtype=dt, device=device)
         ws, nbytes = self._workspace(device, dt, n)
-        _lib.check(plan.lib.spect_forward(plan.handle, _lib.dtype_code(dt), f.data_ptr(), _lib.ptr(m),
+        _lib.check(plan.lib.spect_forward(plan.handle, self._code(dt, None, True), f.data_ptr(), _lib.ptr(m),
                                           None, idx.data_ptr(), n, out.data_ptr(), ws.data_ptr(),
                                           nbytes, _lib.stream_ptr(device)))
         return out

@@ -96,6 +96,17 @@ class UnrolledBSREM:
             ratio.data_ptr(), hf.numel(), float(pytomography_amd.delta), _lib.stream_ptr(hf.device)))
         return pred, ratio
 
+    # The iterations and their derivative blur every plane with its own PSF, as
+    # backward_transpose does: the operators that are differentiated are the
+    # ones that are applied.
+    def _forward(self, x, k):
+        return self.sm._project(x, k, "spect_forward", planes=True) if self.sm.fused else self.sm.forward(x, k)
+
+    def _backward(self, p, k, mode=_lib.BP_REFERENCE):
+        if not self.sm.fused:
+            return self.sm.backward(p, k) if mode == _lib.BP_REFERENCE else self.sm.backward_adjoint(p, k)
+        return self.sm._backward(p, k, mode, planes=True)
+
     def _subset_proj(self, t, k):
         return t if k is None else self.sm.get_projection_subset(t, k).contiguous()
 
@@ -114,9 +125,9 @@ class UnrolledBSREM:
                 ckpts.append(x.clone())
                 w = self._weight(k)
                 r = self.prior.gradient(x, beta_scale=w, beta=beta)
-                hf = self.sm.forward(x, k)
+                hf = self._forward(x, k)
                 _, ratio = self._ratio(self._subset_proj(g, k), hf, self._subset_proj(s, k))
-                b = self.sm.backward(ratio, k)
+                b = self._backward(ratio, k)
                 nk = norms[0 if k is None else k]
                 _lib.check(_lib.lib().spect_bsrem_update(
                     _lib.dtype_code(dt), x.data_ptr(), b.data_ptr(), nk.data_ptr(),
@@ -141,9 +152,9 @@ class UnrolledBSREM:
             w = self._weight(k)
             g_m, s_m = self._subset_proj(g, k), self._subset_proj(s, k)
             r = self.prior.gradient(x, beta_scale=w, beta=beta)
-            hf = self.sm.forward(x, k)
+            hf = self._forward(x, k)
             pred, ratio = self._ratio(g_m, hf, s_m)
-            b = self.sm.backward(ratio, k)
+            b = self._backward(ratio, k)
             nk = norms[0 if k is None else k]
             d = self._precond(j, k, total)
             pre = x * d
@@ -160,7 +171,7 @@ class UnrolledBSREM:
                 idx = self.sm._angle_index(k, device).long()
                 gbar.index_add_(0, idx, gt)
             q = (-(g_m * gt) / p).contiguous()
-            lam = mu * (1 + d * G) + self.sm.backward_adjoint(q, k) \
+            lam = mu * (1 + d * G) + self._backward(q, k, _lib.BP_ADJOINT) \
                 - self.prior.hessian_vjp(x, v, beta_scale=w, beta=beta)
             if beta != 0:
                 betabar -= (v.double() * r.double()).sum() / beta
