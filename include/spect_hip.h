@@ -191,6 +191,13 @@ int spect_backward(const spect_plan *p, int dtype, int mode, int out_mode, const
                    void *out, const void *f, const void *norm, double delta, double floor_value,
                    void *workspace, size_t workspace_bytes, void *stream);
 
+/* Sensitivity image: spect_backward(REFERENCE, STORE) of a projection of ones,
+ * in float64 (dtype SPECT_F64, optionally with SPECT_ATT_FIELD), without
+ * blurring a projection.                                              */
+int spect_sensitivity(const spect_plan *p, int dtype, const void *mu, const void *att_table,
+                      const int32_t *angle_idx, int n, void *out, void *workspace,
+                      size_t workspace_bytes, void *stream);
+
 /* Transpose of the reference back projection: proj = B_m^T v with
  * B_m = spect_backward(REFERENCE) (spect_system_matrix.py:159-201), i.e. the
  * forward projector with the rotation replaced by the transpose of the

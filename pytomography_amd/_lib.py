@@ -29,7 +29,7 @@ EXPORTED = (
     "spect_att_table_bytes", "spect_att_table_build",
     "spect_att_field_bytes", "spect_att_field_build",
     "spect_forward", "spect_forward_noalloc", "spect_backward", "spect_backward_transpose",
-    "spect_osem_subiteration",
+    "spect_sensitivity", "spect_osem_subiteration",
     "spect_grad_workspace_bytes", "spect_forward_vjp",
     "spect_batch_create", "spect_batch_run", "spect_batch_destroy",
     "spect_poisson_ratio", "spect_rdp_gradient", "spect_rdp_hessian_vjp", "spect_rdp_hessian_jvp",
@@ -107,6 +107,8 @@ def _declare(lib):
     lib.spect_forward_noalloc.argtypes = [vp, ci, vp, vp, vp, vp, ci, vp, vp]
     lib.spect_backward.restype = ci
     lib.spect_backward.argtypes = [vp, ci, ci, ci, vp, vp, vp, vp, ci, vp, vp, vp, dbl, dbl, vp, sz, vp]
+    lib.spect_sensitivity.restype = ci
+    lib.spect_sensitivity.argtypes = [vp, ci, vp, vp, vp, ci, vp, vp, sz, vp]
     lib.spect_osem_subiteration.restype = ci
     lib.spect_osem_subiteration.argtypes = [vp, ci, vp, vp, vp, vp, ci, vp, vp, vp, vp, dbl, dbl, vp, sz, vp]
     lib.spect_grad_workspace_bytes.restype = sz

@@ -238,6 +238,7 @@ Ws ws_layout(const spect_plan *p, int dtype, int n) {
   l.part_off = att;
   l.w_off = att;  // forward partials are consumed before the field is written
   l.q_off = att + w;
+  if (dtype == SPECT_F64) w += ones_profile_bytes(n, p->P, (int)n_jext, p->Nz);
   if (dtype == SPECT_F32 && p->lr.nseg > 0) {
     part = std::max(part, lr_forward_bytes(p->lr, g, n));
     w += lr_backward_bytes(p->lr, g, n);
@@ -1127,6 +1128,33 @@ int spect_backward(const spect_plan *p, int dtype, int mode, int out_mode, const
   return backward_impl<double>(p, mode, out_mode, (const double *)proj, (const double *)mu,
                                att_table, field, angle_idx, n, (double *)out, (const double *)f,
                                (const double *)norm, delta, floor_value, ws, st);
+}
+
+int spect_sensitivity(const spect_plan *p, int dtype, const void *mu, const void *att_table,
+                      const int32_t *angle_idx, int n, void *out, void *workspace,
+                      size_t workspace_bytes, void *stream) {
+  const bool field = (dtype & SPECT_ATT_FIELD) != 0;
+  dtype &= ~SPECT_ATT_FIELD;
+  if (dtype != SPECT_F64) return fail(SPECT_E_ARG, "dtype must be F64");
+  if (int rc = check_call(p, dtype, n, workspace, workspace_bytes)) return rc;
+  if (!out || !angle_idx) return fail(SPECT_E_ARG, "null array argument");
+  if (int rc = check_arrays({mu, att_table, out})) return rc;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  auto *ws = reinterpret_cast<unsigned char *>(workspace);
+  const Geo<double> g = geo<double>(p);
+  const Ws l = ws_layout(p, dtype, n);
+  const double *att, *attf;
+  bool global;
+  if (int rc = att_rows<double>(p, g, (const double *)mu, att_table, field, angle_idx, n,
+                                reinterpret_cast<double *>(ws + l.att_off), st, &att, &global, &attf))
+    return rc;
+  double *W = reinterpret_cast<double *>(ws + l.w_off);
+  HIP_TRY(launch_ones_field(g, tables<double>(p), (const double *)mu, att, global, attf, angle_idx, n, W,
+                            reinterpret_cast<double *>(ws + l.q_off), st));
+  HIP_TRY(launch_bp_gather<double>(g, tables<double>(p), W, angle_idx, n, SPECT_BP_REFERENCE,
+                                   SPECT_OUT_STORE, (double *)out, nullptr, nullptr, 0.0, 0.0, nullptr,
+                                   nullptr, nullptr, st));
+  return SPECT_OK;
 }
 
 int spect_osem_subiteration(const spect_plan *p, int dtype, void *f, const void *mu,

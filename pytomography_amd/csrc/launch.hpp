@@ -183,6 +183,13 @@ hipError_t launch_bp_gather(const Geo<R> &g, const Tables<R> &tb, const R *W,
                             const double *Pref, R *out_mu, hipStream_t st,
                             size_t w_astride = 0, size_t w_rstride = 0);
 
+// The field of a back projection of ones (sensitivity.hip); prof:
+// ones_profile_bytes.
+size_t ones_profile_bytes(int n, int P, int n_jext, int Nz);
+hipError_t launch_ones_field(const Geo<double> &g, const Tables<double> &tb, const double *mu, const double *att,
+                             bool att_global, const double *attf, const int32_t *angle_idx, int n, double *W,
+                             double *prof, hipStream_t st);
+
 // Elementwise and stencil kernels (misc.hip).
 template <typename R>
 hipError_t launch_ratio(const R *g, const R *hf, const R *s, R *pred, R *ratio, int64_t count,

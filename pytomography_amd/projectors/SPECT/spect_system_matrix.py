@@ -258,12 +258,31 @@ class SPECTSystemMatrix(SystemMatrix):
         """H_m^T 1 (spect_system_matrix.py:106-118), computed in
         ``sensitivity_dtype`` on the GPU and returned in the working dtype."""
         device = pytomography_amd.device
+        if self.fused and self._psf is not None and self.sensitivity_dtype == torch.float64:
+            return self._sensitivity(subset_idx).to(pytomography_amd.dtype)
         n = self.proj_meta.num_projections if subset_idx is None else len(self.subset_indices_array[subset_idx])
         ones = torch.ones((n, *self.proj_meta.shape[1:]), dtype=self.sensitivity_dtype, device=device)
         if not self.fused:
             return self._backward_frames(ones, subset_idx).to(pytomography_amd.dtype)
         out = self._backward(ones, subset_idx, _lib.BP_REFERENCE)
         return out.to(pytomography_amd.dtype)
+
+    def _sensitivity(self, subset_idx) -> torch.Tensor:
+        """Float64 back projection of ones: with a PSF, ``spect_sensitivity`` blurs
+        two profiles instead of every plane (without one, the projection itself
+        is gathered and there is nothing to save)."""
+        device, dt = pytomography_amd.device, torch.float64
+        plan = self._plan(device)
+        idx = self._angle_index(subset_idx, device)
+        n = idx.numel()
+        mu = self._mu(device, dt)
+        tab = self._att_table(device, dt)
+        out = torch.empty(self._shape, dtype=dt, device=device)
+        ws, nbytes = self._workspace(device, dt, n)
+        _lib.check(plan.lib.spect_sensitivity(plan.handle, self._code(dt, tab), _lib.ptr(mu), _lib.ptr(tab),
+                                              idx.data_ptr(), n, out.data_ptr(), ws.data_ptr(), nbytes,
+                                              _lib.stream_ptr(device)))
+        return out
 
     # ------------------------------------------------------------ projections
     def forward(self, object: torch.Tensor, subset_idx: int | None = None) -> torch.Tensor:
