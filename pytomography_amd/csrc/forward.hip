@@ -40,19 +40,19 @@ int tile_block_threads(int Nz, int run_len, int splits) {
 namespace {
 
 template <typename R, int RZ>
-__global__ __launch_bounds__(1024) void att_table_kernel(Geo<R> g, Tables<R> tb,
+__global__ __launch_bounds__(256) void att_table_kernel(Geo<R> g, Tables<R> tb,
                                                         const R *__restrict__ mu,
                                                         const int32_t *__restrict__ angle_idx,
                                                         double *__restrict__ table) {
-  att_table_body<R, RZ>(g, tb, mu, angle_idx, table, blockIdx.x, blockIdx.y);
+  att_table_body<R, RZ>(g, tb, mu, angle_idx, table, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
 template <typename R, int RZ>
-__global__ __launch_bounds__(1024) void att_field_kernel(Geo<R> g, Tables<R> tb,
+__global__ __launch_bounds__(256) void att_field_kernel(Geo<R> g, Tables<R> tb,
                                                         const R *__restrict__ mu,
                                                         const int32_t *__restrict__ angle_idx,
                                                         R *__restrict__ field) {
-  att_field_body<R, RZ>(g, tb, mu, angle_idx, field, blockIdx.x, blockIdx.y);
+  att_field_body<R, RZ>(g, tb, mu, angle_idx, field, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
 template <typename R, int RZ, int QS, int H, bool TRB, bool AF>
@@ -244,22 +244,18 @@ hipError_t launch_reduce_sched(const Geo<R> &g, const R *partial, int n, const i
 template <typename R>
 hipError_t launch_att_table(const Geo<R> &g, const Tables<R> &tb, const R *mu,
                             const int32_t *angle_idx, int n, double *table, hipStream_t st) {
-  constexpr int RZ = FwdTile<R>::RZ;
-  const int runs = (g.Nz + RZ - 1) / RZ;
-  const int bt = (kTJ * runs + 63) / 64 * 64;
-  dim3 grid(n, g.ntiles);
-  att_table_kernel<R, RZ><<<grid, bt, 0, st>>>(g, tb, mu, angle_idx, table);
+  constexpr int RZ = 16 / sizeof(R);  // a 16-byte load per sample row
+  const int items = min(kTJ, g.je1 - g.je0) * ((g.Nz + RZ - 1) / RZ);
+  att_table_kernel<R, RZ><<<dim3(n, g.ntiles, (items + 255) / 256), 256, 0, st>>>(g, tb, mu, angle_idx, table);
   return hipGetLastError();
 }
 
 template <typename R>
 hipError_t launch_att_field(const Geo<R> &g, const Tables<R> &tb, const R *mu,
                             const int32_t *angle_idx, int n, R *field, hipStream_t st) {
-  constexpr int RZ = FwdTile<R>::RZ;
-  const int runs = (g.Nz + RZ - 1) / RZ;
-  const int bt = (kTJ * runs + 63) / 64 * 64;
-  dim3 grid(n, g.ntiles);
-  att_field_kernel<R, RZ><<<grid, bt, 0, st>>>(g, tb, mu, angle_idx, field);
+  constexpr int RZ = 16 / sizeof(R);  // a 16-byte load per sample row
+  const int items = min(kTJ, g.je1 - g.je0) * ((g.Nz + RZ - 1) / RZ);
+  att_field_kernel<R, RZ><<<dim3(n, g.ntiles, (items + 255) / 256), 256, 0, st>>>(g, tb, mu, angle_idx, field);
   return hipGetLastError();
 }
 

@@ -11,116 +11,110 @@
 
 namespace spect {
 
-// Attenuation march of one (angle al, 32-column tile jt) block, grid (n, ntiles).
-template <typename R, int RZ>
-__device__ __forceinline__ void att_table_body(const Geo<R> &g, const Tables<R> &tb,
-                                               const R *__restrict__ mu,
-                                               const int32_t *__restrict__ angle_idx,
-                                               double *__restrict__ table, int al, int jt) {
-  __shared__ Src<R> src[kTJ];
-  const int ang = ld_uniform(angle_idx + al);
-  if ((unsigned)ang >= (unsigned)g.A) return;
-  const int tid = threadIdx.x;
-  const int j0 = g.je0 + jt * kTJ;
-  const int tj = min(kTJ, g.je1 - j0);
+// Attenuation march of angle al and 32-column tile jt, from the detector's side
+// (plane P - 1) down: plane(i, S, xm) after every plane, for the lane's RZ
+// consecutive z of one column, with the FP64 sum S of the planes so far and the
+// plane's own mu dx.  Lanes run along z, then along the columns; no lane waits
+// for another, and the samples of four planes are requested together, since a
+// lane's loads are a serial chain otherwise (the sums are in the planes' order).
+// Samples outside the footprint have zero weights: a group of planes that no
+// lane of the wave samples is skipped.  part of parts: blocks of a tile.
+// Latency bounds it: one run of 16 z per lane and a barrier per plane left about
+// one wave per SIMD (487 us for the table of 60 angles at 128^3; now 144).
+template <typename R, int RZ, typename Plane>
+__device__ __forceinline__ void att_march(const Geo<R> &g, const Tables<R> &tb, const R *__restrict__ mu,
+                                          int ang, int jt, int part, int parts, Plane plane) {
+  constexpr int U = 4;  // planes in flight
+  const int j0 = g.je0 + jt * kTJ, tj = min(kTJ, g.je1 - j0);
   const int runs = (g.Nz + RZ - 1) / RZ;
-  const int jl = tid % kTJ, run = tid / kTJ, z0 = run * RZ;
-  const bool mine = run < runs && jl < tj;
-  const int n_jext = g.je1 - g.je0;
   const auto cs = ld_uniform(tb.trig + ang);
-  double S[RZ];
+  for (int q = part * blockDim.x + threadIdx.x; q < tj * runs; q += parts * blockDim.x) {
+    const int jl = q / runs, z0 = (q - jl * runs) * RZ;
+    const R lin = tb.lin[j0 + jl];
+    double S[RZ];
 #pragma unroll
-  for (int m = 0; m < RZ; ++m) S[m] = 0.0;
-  auto row = [&](int c, int m) -> size_t {
-    return (((size_t)al * g.C + c) * n_jext + (j0 - g.je0 + jl)) * g.Nz + z0 + m;
-  };
-  if (mine) {
+    for (int m = 0; m < RZ; ++m) S[m] = 0.0;
+    for (int i0 = g.P - 1; i0 >= 0; i0 -= U) {
+      R x[U][RZ];
+      Taps4<R> t[U];
+      bool inside = false;
 #pragma unroll
-    for (int m = 0; m < RZ; ++m)
-      if (z0 + m < g.Nz) table[row(g.C - 1, m)] = 0.0;
-  }
-  for (int i = g.P - 1; i >= 0; --i) {
-    int inside = 0;
-    if (tid < tj) {
-      R ix, iy;
-      rot_coord<R>(cs.x, cs.y, tb.lin[j0 + tid], ld_uniform(tb.lin + i), g.half, ix, iy);
-      src[tid] = make_src<R>(ix, iy, g.pad);
-      inside = in_footprint<R>(ix, iy, g);
-    }
-    if (__syncthreads_or(inside)) {
-      if (mine) {
-        const Taps4<R> t = taps4<R>(src[jl], g.N, g.Nz);
-        R x[RZ];
-        gather_run<R, RZ>(mu, t, z0, g.Nz, x);
-#pragma unroll
-        for (int m = 0; m < RZ; ++m) S[m] += (double)(x[m] * g.dx);
+      for (int k = 0; k < U; ++k) {
+        R ix, iy;
+        rot_coord<R>(cs.x, cs.y, lin, tb.lin[max(i0 - k, 0)], g.half, ix, iy);
+        t[k] = taps4<R>(make_src<R>(ix, iy, g.pad), g.N, g.Nz);
+        inside = inside || in_footprint<R>(ix, iy, g);
       }
-      __syncthreads();  // src is rewritten by the next plane
-    }
-    if (mine && i > 0 && i % g.L == 0) {
-      const int c = i / g.L - 1;
+      if (inside) {
 #pragma unroll
-      for (int m = 0; m < RZ; ++m)
-        if (z0 + m < g.Nz) table[row(c, m)] = S[m];
+        for (int k = 0; k < U; ++k) gather_run<R, RZ>(mu, t[k], z0, g.Nz, x[k]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+#pragma unroll
+          for (int m = 0; m < RZ; ++m) x[k][m] = R(0);
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        if (i0 - k < 0) continue;
+#pragma unroll
+        for (int m = 0; m < RZ; ++m) {
+          x[k][m] = x[k][m] * g.dx;
+          S[m] += (double)x[k][m];
+        }
+        plane(i0 - k, jl, z0, S, x[k]);
+      }
     }
   }
 }
 
+// The suffix table: row c holds the sum over the planes above chunk c.
+template <typename R, int RZ>
+__device__ __forceinline__ void att_table_body(const Geo<R> &g, const Tables<R> &tb,
+                                               const R *__restrict__ mu,
+                                               const int32_t *__restrict__ angle_idx,
+                                               double *__restrict__ table, int al, int jt,
+                                               int part = 0, int parts = 1) {
+  const int ang = ld_uniform(angle_idx + al);
+  if ((unsigned)ang >= (unsigned)g.A) return;
+  const int n_jext = g.je1 - g.je0;
+  auto store = [&](int c, int jl, int z0, const double (&v)[RZ]) {
+    double *dst = table + (((size_t)al * g.C + c) * n_jext + (jt * kTJ + jl)) * g.Nz + z0;
+#pragma unroll
+    for (int m = 0; m < RZ; ++m)
+      if (z0 + m < g.Nz) dst[m] = v[m];
+  };
+  att_march<R, RZ>(g, tb, mu, ang, jt, part, parts,
+                   [&](int i, int jl, int z0, const double (&S)[RZ], const R (&)[RZ]) {
+                     if (i == g.P - 1) {
+                       double zero[RZ] = {};
+                       store(g.C - 1, jl, z0, zero);
+                     }
+                     if (i > 0 && i % g.L == 0) store(i / g.L - 1, jl, z0, S);
+                   });
+}
+
 // The attenuation factor itself, a(i, j, z) = exp(-(S(i) - x(i)/2)) in R, for
-// every plane whose tile footprint is non-empty (the planes the projection
-// kernels visit), from the same FP64 march as att_table_kernel: the forward
-// and field kernels then read it instead of gathering mu (bitwise the same
-// factors).  field layout: [angle][P][je1-je0][Nz].
+// every plane (also where a column samples no object: the projectors may visit
+// a plane a conservative activity test keeps), from the same FP64 march as the
+// table: the forward and field kernels then read it instead of gathering mu
+// (bitwise the same factors).  field layout: [angle][P][je1-je0][Nz].
 template <typename R, int RZ>
 __device__ __forceinline__ void att_field_body(const Geo<R> &g, const Tables<R> &tb,
                                                const R *__restrict__ mu,
                                                const int32_t *__restrict__ angle_idx,
-                                               R *__restrict__ field, int al, int jt) {
-  __shared__ Src<R> src[kTJ];
+                                               R *__restrict__ field, int al, int jt,
+                                               int part = 0, int parts = 1) {
   const int ang = ld_uniform(angle_idx + al);
   if ((unsigned)ang >= (unsigned)g.A) return;
-  const int tid = threadIdx.x;
-  const int j0 = g.je0 + jt * kTJ;
-  const int tj = min(kTJ, g.je1 - j0);
-  const int runs = (g.Nz + RZ - 1) / RZ;
-  const int jl = tid % kTJ, run = tid / kTJ, z0 = run * RZ;
-  const bool mine = run < runs && jl < tj;
   const int n_jext = g.je1 - g.je0;
-  const auto cs = ld_uniform(tb.trig + ang);
-  double S[RZ];
+  att_march<R, RZ>(g, tb, mu, ang, jt, part, parts,
+                   [&](int i, int jl, int z0, const double (&S)[RZ], const R (&xm)[RZ]) {
+                     R *dst = field + (((size_t)al * g.P + i) * n_jext + (jt * kTJ + jl)) * g.Nz + z0;
 #pragma unroll
-  for (int m = 0; m < RZ; ++m) S[m] = 0.0;
-  for (int i = g.P - 1; i >= 0; --i) {
-    int inside = 0;
-    if (tid < tj) {
-      R ix, iy;
-      rot_coord<R>(cs.x, cs.y, tb.lin[j0 + tid], ld_uniform(tb.lin + i), g.half, ix, iy);
-      src[tid] = make_src<R>(ix, iy, g.pad);
-      inside = in_footprint<R>(ix, iy, g);
-    }
-    // Every plane gets its factors, also where the tile samples no object
-    // (mu is zero there, so S carries over): the projectors may visit a
-    // plane a conservative activity test keeps.
-    const bool any = __syncthreads_or(inside);
-    if (mine) {
-      R x[RZ];
-      if (any) {
-        const Taps4<R> t = taps4<R>(src[jl], g.N, g.Nz);
-        gather_run<R, RZ>(mu, t, z0, g.Nz, x);
-      } else {
-#pragma unroll
-        for (int m = 0; m < RZ; ++m) x[m] = R(0);
-      }
-      R *dst = field + (((size_t)al * g.P + i) * n_jext + (j0 - g.je0 + jl)) * g.Nz + z0;
-#pragma unroll
-      for (int m = 0; m < RZ; ++m) {
-        const R xm = x[m] * g.dx;
-        S[m] += (double)xm;
-        if (z0 + m < g.Nz) dst[m] = att_factor<R>(S[m], xm);
-      }
-    }
-    __syncthreads();  // src is rewritten by the next plane
-  }
+                     for (int m = 0; m < RZ; ++m)
+                       if (z0 + m < g.Nz) dst[m] = att_factor<R>(S[m], xm[m]);
+                   });
 }
 
 // LDS rows: H zeros | runs*RZ values | H zeros | 1 pad (odd stride).

@@ -3,8 +3,9 @@
 // A plane's PSF is separable, so the blur of a constant projection is the outer
 // product of two profiles: W(i,j,z) = a(i,j,z) u_i(j) v_i(z), u_i and v_i the
 // sums of the taps that fall on the detector.  No plane is blurred: what is left
-// is the attenuation march and the store of W.  15 angles at 128^3 with the
-// suffix table: PENDING us against 860 for blurring a projection of ones.
+// is the attenuation march and the store of W, 8 bytes a sample.  8 angles at
+// 128^3 with the suffix table: 61 us, against 451 us for blurring a projection
+// of ones.
 #include <type_traits>
 
 #include "launch.hpp"
