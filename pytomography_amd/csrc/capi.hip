@@ -340,10 +340,12 @@ int forward_core(const spect_plan *p, const R *f, const R *mu, const void *table
       if (lr_forward_bytes(p->lr, g, k) <= part_bytes) {
         const size_t rows_n = (size_t)(g.jo1 - g.jo0) * g.Nz;
         auto at = [&](auto *q, size_t a) { return q ? q + a * rows_n : q; };
-        for (int a = 0; a < n; a += k)
-          HIP_TRY(launch_lr_forward(g, tables<R>(p), p->lr, f, attf, idx + a, std::min(k, n - a), at(proj, a),
-                                    at(gm, a), at(s, a), at(pred, a), at(ratio, a), delta,
-                                    reinterpret_cast<unsigned char *>(part), part_bytes, st));
+        for (int a = 0; a < n; a += k) {
+          const LrGatherJob J = lr_gather_job(g, tables<R>(p), p->lr, f, attf, idx + a, std::min(k, n - a),
+                                              reinterpret_cast<unsigned char *>(part));
+          HIP_TRY(launch_lr_forward(J, lr_blur_job(J, at(proj, a), at(gm, a), at(s, a), at(pred, a), at(ratio, a), delta),
+                                    part_bytes, st));
+        }
         return SPECT_OK;
       }
     }
@@ -398,7 +400,8 @@ int backward_impl(const spect_plan *p, int mode, int out_mode, const R *proj, co
   R *W = reinterpret_cast<R *>(ws + l.w_off);
   if constexpr (sizeof(R) == 4) {
     if (!planes && lr_runs(p, attf, mu) && lr_back_pays(g, n)) {
-      HIP_TRY(launch_lr_field(g, tables<R>(p), p->lr, proj, attf, idx, n, W, ws + l.q_off, l.ratio_off - l.q_off, st));
+      HIP_TRY(launch_lr_field(lr_back_job(g, tables<R>(p), p->lr, proj, attf, idx, n, W, ws + l.q_off),
+                              l.ratio_off - l.q_off, st));
       HIP_TRY(launch_bp_gather<R>(g, tables<R>(p), W, idx, n, mode, out_mode, out, f, nrm, R(delta),
                                   R(floor_value), nullptr, nullptr, nullptr, st));
       return SPECT_OK;
@@ -463,6 +466,11 @@ struct spect_batch {
     // per subset: device offsets (bytes) into `tables` and block counts
     std::vector<size_t> fwd_off, red_off, fld_off, gat_off, starts_off[4];
     std::vector<int> blocks[4];
+    // members that blur combined images: their descriptors per subset, and the
+    // device offsets of the jobs and starts
+    bool images = false;
+    std::vector<LrBatch> lr;
+    std::vector<size_t> lr_off[3], lr_starts[4];
   };
   std::vector<Group> groups;
   void *tables = nullptr;  // device: job arrays and block starts
@@ -477,6 +485,12 @@ struct spect_batch {
 
 namespace {
 
+// Whether a batched problem blurs combined images, as its single calls do.
+template <typename R> bool batch_images(const spect_batch_problem &pb) {
+  if constexpr (sizeof(R) == 4) return pb.plan->lr.nseg > 0 && (pb.att_field || !pb.mu);
+  else return false;
+}
+
 template <typename R>
 int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double delta,
                 double floor_value) {
@@ -484,9 +498,10 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
   std::vector<std::vector<int>> members;
   std::vector<std::pair<int, int>> keys;
   for (int i = 0; i < n; ++i) {
-    // the key packs (H, attenuation-field flag) and Nz
-    const std::pair<int, int> key{probs[i].plan->H * 2 + (probs[i].att_field ? 1 : 0),
-                                  probs[i].plan->Nz};
+    // the key packs (H, combined images, attenuation-field flag) and Nz
+    const std::pair<int, int> key{
+        probs[i].plan->H * 4 + (batch_images<R>(probs[i]) ? 2 : 0) + (probs[i].att_field ? 1 : 0),
+        probs[i].plan->Nz};
     size_t k = 0;
     while (k < keys.size() && keys[k] != key) ++k;
     if (k == keys.size()) {
@@ -512,7 +527,8 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
   };
   for (size_t k = 0; k < keys.size(); ++k) {
     spect_batch::Group G;
-    G.H = keys[k].first / 2;
+    G.H = keys[k].first / 4;
+    G.images = (keys[k].first & 2) != 0;
     G.af = (keys[k].first & 1) != 0;
     G.Nz = keys[k].second;
     G.nprob = (int)members[k].size();
@@ -525,6 +541,7 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
       std::vector<GatherJob<R>> gj;
       std::vector<int> st[4];
       int tot[4] = {0, 0, 0, 0};
+      LrBatch lb;
       for (int i : members[k]) {
         const spect_batch_problem &pb = probs[i];
         const spect_plan *p = pb.plan;
@@ -550,12 +567,29 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
         gj.push_back(GatherJob<R>{g, tb, W, idx, cnt, SPECT_OUT_OSEM, f, f,
                                   reinterpret_cast<const R *>(pb.norm[sub]), R(delta),
                                   R(floor_value), nullptr, nullptr, nullptr});
+        if constexpr (sizeof(R) == 4) {
+          if (G.images) {
+            const LrGatherJob J = lr_gather_job(g, tb, p->lr, f, attf, idx, cnt, ws + l.part_off);
+            lb.gather.push_back(J);
+            lb.blur.push_back(lr_blur_job(J, nullptr, rj.back().gm, rj.back().s, rj.back().pred, ratio, R(delta)));
+            lb.back.push_back(lr_back_job(g, tb, p->lr, ratio, attf, idx, cnt, W, ws + l.q_off));
+          }
+        }
         const int nb[4] = {fwd_blocks(g, cnt), reduce_blocks(g, cnt), fwd_blocks(g, cnt),
                            gather_blocks(g)};
         for (int q = 0; q < 4; ++q) {
           st[q].push_back(tot[q]);
           tot[q] += nb[q];
         }
+      }
+      if (G.images) {
+        if (!lr_batch_finish(lb)) return fail(SPECT_E_ARG, "batch too large");
+        G.lr_off[0].push_back(put(lb.gather.data(), lb.gather.size() * sizeof(lb.gather[0])));
+        G.lr_off[1].push_back(put(lb.blur.data(), lb.blur.size() * sizeof(lb.blur[0])));
+        G.lr_off[2].push_back(put(lb.back.data(), lb.back.size() * sizeof(lb.back[0])));
+        for (int q = 0; q < 4; ++q)
+          G.lr_starts[q].push_back(put(lb.starts[q].data(), lb.starts[q].size() * sizeof(int)));
+        G.lr.push_back(std::move(lb));
       }
       G.fwd_off.push_back(put(fj.data(), fj.size() * sizeof(fj[0])));
       G.red_off.push_back(put(rj.data(), rj.size() * sizeof(rj[0])));
@@ -581,15 +615,24 @@ int batch_launch_group(spect_batch *b, const spect_batch::Group &G, int n_iters,
   auto *base = reinterpret_cast<unsigned char *>(b->tables);
   for (int it = 0; it < n_iters; ++it) {
     for (int sub = 0; sub < b->n_subsets; ++sub) {
-      HIP_TRY(launch_forward_batch<R>(reinterpret_cast<const FwdJob<R> *>(base + G.fwd_off[sub]),
-                                      reinterpret_cast<const int *>(base + G.starts_off[0][sub]),
-                                      G.nprob, G.blocks[0][sub], G.H, G.Nz, G.maxL, G.af, st));
-      HIP_TRY(launch_reduce_batch<R>(reinterpret_cast<const ReduceJob<R> *>(base + G.red_off[sub]),
-                                     reinterpret_cast<const int *>(base + G.starts_off[1][sub]),
-                                     G.nprob, G.blocks[1][sub], st));
-      HIP_TRY(launch_field_batch<R>(reinterpret_cast<const FieldJob<R> *>(base + G.fld_off[sub]),
-                                    reinterpret_cast<const int *>(base + G.starts_off[2][sub]),
-                                    G.nprob, G.blocks[2][sub], G.H, G.Nz, G.maxL, G.af, st));
+      if (G.images) {
+        auto starts = [&](int q) { return reinterpret_cast<const int *>(base + G.lr_starts[q][sub]); };
+        HIP_TRY(launch_lr_batch_forward(G.lr[sub], reinterpret_cast<const LrGatherJob *>(base + G.lr_off[0][sub]),
+                                        reinterpret_cast<const LrBlurJob *>(base + G.lr_off[1][sub]), starts(0),
+                                        starts(1), st));
+        HIP_TRY(launch_lr_batch_field(G.lr[sub], reinterpret_cast<const LrBackJob *>(base + G.lr_off[2][sub]),
+                                      starts(2), starts(3), st));
+      } else {
+        HIP_TRY(launch_forward_batch<R>(reinterpret_cast<const FwdJob<R> *>(base + G.fwd_off[sub]),
+                                        reinterpret_cast<const int *>(base + G.starts_off[0][sub]),
+                                        G.nprob, G.blocks[0][sub], G.H, G.Nz, G.maxL, G.af, st));
+        HIP_TRY(launch_reduce_batch<R>(reinterpret_cast<const ReduceJob<R> *>(base + G.red_off[sub]),
+                                       reinterpret_cast<const int *>(base + G.starts_off[1][sub]),
+                                       G.nprob, G.blocks[1][sub], st));
+        HIP_TRY(launch_field_batch<R>(reinterpret_cast<const FieldJob<R> *>(base + G.fld_off[sub]),
+                                      reinterpret_cast<const int *>(base + G.starts_off[2][sub]),
+                                      G.nprob, G.blocks[2][sub], G.H, G.Nz, G.maxL, G.af, st));
+      }
       HIP_TRY(launch_gather_batch<R>(reinterpret_cast<const GatherJob<R> *>(base + G.gat_off[sub]),
                                      reinterpret_cast<const int *>(base + G.starts_off[3][sub]),
                                      G.nprob, G.blocks[3][sub], SPECT_BP_REFERENCE, st));

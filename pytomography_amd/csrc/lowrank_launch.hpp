@@ -2,6 +2,8 @@
 // combined images (lowrank_body.hpp, lowrank.hip).
 #pragma once
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace spect {
@@ -101,10 +103,12 @@ inline int lr_gather_zgroups(const Geo<float> &g) {
 // OSEM, cached / streamed: 128^3 x 120 angles 1743 / 1638 us, 192^3 x 180 8283 /
 // 8099, 100^2 x 47 655 / 731, 64^3 x 60 518 / 528.
 constexpr int kLrCached = 1, kLrStream = 2;
-inline int lr_factor_mode(const Geo<float> &g, const float *attf) {
+inline int lr_factor_mode(int Nz, const float *attf, size_t field_bytes) {
   if (!attf) return 0;
-  const size_t field = (size_t)g.A * g.P * (g.je1 - g.je0) * g.Nz * sizeof(float);
-  return g.Nz % 32 != 0 || field <= (size_t)256 << 20 ? kLrCached : kLrStream;
+  return Nz % 32 != 0 || field_bytes <= (size_t)256 << 20 ? kLrCached : kLrStream;
+}
+inline int lr_factor_mode(const Geo<float> &g, const float *attf) {
+  return lr_factor_mode(g.Nz, attf, (size_t)g.A * g.P * (g.je1 - g.je0) * g.Nz * sizeof(float));
 }
 
 // An image is stored in tiles of 16 columns j x 16 z, the blurs' unit, each
@@ -125,14 +129,7 @@ __host__ __device__ inline uint32_t lr_image_at(const Geo<float> &g, int NzP, in
 // First tile row that holds an extended column, and tile rows from it to the last.
 __host__ __device__ inline int lr_first_tile(const Geo<float> &g) { return kLrLead - (g.jo0 - g.je0 + 15) / 16; }
 inline int lr_back_rows(const Geo<float> &g) { return (g.jo0 - g.je0 + 15) / 16 + (g.je1 - g.jo0 + 15) / 16; }
-inline int lr_back_tiles(const Geo<float> &g, int n) {
-  return (long long)n * ((lr_back_rows(g) + kLrBackTiles - 1) / kLrBackTiles) * (lr_nzp(g.Nz) / 16) >= 192 ? kLrBackTiles
-                                                                                               : kLrBackTilesFew;
-}
-inline int lr_back_ranges(const Geo<float> &g, int n) {
-  const int nt = lr_back_tiles(g, n);
-  return (lr_back_rows(g) + nt - 1) / nt;
-}
+inline int lr_back_ranges(const Geo<float> &g, int nt) { return (lr_back_rows(g) + nt - 1) / nt; }
 // Row tiles after the last image that the forward's blur may read (and ignore).
 constexpr int kLrPadTiles = kLrRowTiles;
 
@@ -152,19 +149,42 @@ inline size_t lr_forward_bytes(const LrTables &lr, const Geo<float> &g, int n) {
 inline size_t lr_backward_image_bytes(const LrTables &lr, const Geo<float> &g, int n) {
   return lr_image_bytes(lr, g, n);
 }
+// (flags for the most ranges, so that a launch may choose its tiles)
 inline size_t lr_backward_bytes(const LrTables &lr, const Geo<float> &g, int n) {
   return lr_backward_image_bytes(lr, g, n) +
-         lr_align((size_t)n * lr_back_ranges(g, n) * (lr_nzp(g.Nz) / 16) * sizeof(int32_t));
+         lr_align((size_t)n * lr_back_ranges(g, kLrBackTilesFew) * (lr_nzp(g.Nz) / 16) * sizeof(int32_t));
 }
 
-// scratch: lr_forward_bytes / lr_backward_bytes; a smaller one is refused.
-hipError_t launch_lr_forward(const Geo<float> &g, const Tables<float> &tb, const LrTables &lr, const float *f,
-                             const float *attf, const int32_t *angle_idx, int n, float *proj,
-                             const float *gm, const float *s, float *pred, float *ratio, float delta,
-                             unsigned char *scratch, size_t scratch_bytes, hipStream_t st);
-// W[n][P][je1-je0][Nz], every entry that the gathers read.
-hipError_t launch_lr_field(const Geo<float> &g, const Tables<float> &tb, const LrTables &lr, const float *proj,
-                           const float *attf, const int32_t *angle_idx, int n, float *W, unsigned char *scratch,
-                           size_t scratch_bytes, hipStream_t st);
+// The descriptors of one call.  scratch: lr_forward_bytes / lr_backward_bytes.
+LrGatherJob lr_gather_job(const Geo<float> &g, const Tables<float> &tb, const LrTables &lr, const float *f,
+                          const float *attf, const int32_t *angle_idx, int n, unsigned char *scratch);
+LrBlurJob lr_blur_job(const LrGatherJob &J, float *proj, const float *gm, const float *s, float *pred, float *ratio,
+                      float delta);
+// W[n][P][je1-je0][Nz], every entry that the gathers read
+LrBackJob lr_back_job(const Geo<float> &g, const Tables<float> &tb, const LrTables &lr, const float *proj,
+                      const float *attf, const int32_t *angle_idx, int n, float *W, unsigned char *scratch);
+
+// Scratch smaller than that is refused.
+hipError_t launch_lr_forward(const LrGatherJob &J, const LrBlurJob &B, size_t scratch_bytes, hipStream_t st);
+hipError_t launch_lr_field(LrBackJob J, size_t scratch_bytes, hipStream_t st);
+
+// The four passes of several calls with one Nz and one class of half widths
+// (H <= 16 or not), all with attenuation factors or all without, in one launch
+// each.
+struct LrBatch {
+  std::vector<LrGatherJob> gather;
+  std::vector<LrBlurJob> blur;
+  std::vector<LrBackJob> back;
+  std::vector<int> starts[4];  // first block of each call: gather, blur, back blur, field
+  int blocks[4];
+  int row_tiles, back_tiles, waves, factor_mode, H, Nz;
+};
+// Fills everything that follows from gather, blur and back.
+bool lr_batch_finish(LrBatch &b);
+// Descriptors and starts in device memory.
+hipError_t launch_lr_batch_forward(const LrBatch &b, const LrGatherJob *gather, const LrBlurJob *blur,
+                                   const int *gather_starts, const int *blur_starts, hipStream_t st);
+hipError_t launch_lr_batch_field(const LrBatch &b, const LrBackJob *back, const int *blur_starts,
+                                 const int *field_starts, hipStream_t st);
 
 }  // namespace spect
