@@ -59,8 +59,8 @@ class SPECTSystemMatrix(SystemMatrix):
         object_initial_based_on_camera_path: not supported (must be False).
         sensitivity_dtype: dtype of the H^T 1 computation (float64 default).
         chunk_planes: planes per uniform work chunk (0: library default, 16).
-        sched_rounds: the forward projection and the back projection's field
-            kernel, without attenuation or with the attenuation field, split
+        sched_rounds: for calls that blur every plane (float64, no PSF, derivatives):
+            the forward projection and the back projection's field kernel, without attenuation or with the attenuation field, split
             their visited planes evenly over this many rounds of the blocks the
             GPU holds at once; 0 (default) chooses per call: one round when the
             call's pieces of at most 32 planes fit the resident blocks (for the
