@@ -98,13 +98,22 @@ class UnrolledBSREM:
 
     # The iterations and their derivative blur every plane with its own PSF, as
     # backward_transpose does: the operators that are differentiated are the
-    # ones that are applied.
+    # ones that are applied.  (A system matrix with projections of its own, or
+    # on the per-angle path, is called as it is.)
+    def _own(self, name) -> bool:
+        from pytomography_amd.projectors.SPECT import SPECTSystemMatrix
+        return (getattr(type(self.sm), name, None) is not getattr(SPECTSystemMatrix, name)
+                or not self.sm.fused)
+
     def _forward(self, x, k):
-        return self.sm._project(x, k, "spect_forward", planes=True) if self.sm.fused else self.sm.forward(x, k)
+        if self._own("forward"):
+            return self.sm.forward(x, k)
+        return self.sm._project(x, k, "spect_forward", planes=True)
 
     def _backward(self, p, k, mode=_lib.BP_REFERENCE):
-        if not self.sm.fused:
-            return self.sm.backward(p, k) if mode == _lib.BP_REFERENCE else self.sm.backward_adjoint(p, k)
+        name = "backward" if mode == _lib.BP_REFERENCE else "backward_adjoint"
+        if self._own(name):
+            return getattr(self.sm, name)(p, k)
         return self.sm._backward(p, k, mode, planes=True)
 
     def _subset_proj(self, t, k):
