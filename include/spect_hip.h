@@ -49,8 +49,7 @@ enum { SPECT_ATT_FIELD = 0x100 };
 
 /* Flag OR-ed into the dtype argument of spect_forward and spect_backward: blur
  * every plane with its own PSF, as the transposes and derivatives of those calls
- * do, where a float32 call may otherwise blur a few combined images that
- * represent the planes' PSFs to 2^-22. */
+ * do, also with a plan of spect_plan_create_images (any other plan always does). */
 enum { SPECT_PLANES = 0x200 };
 
 /* Padding modes of spect_smooth_axis (torch Conv1d padding_mode). */
@@ -106,6 +105,17 @@ int spect_version(void);
 
 /* Build a plan: uploads trig, linspace and PSF tables to the current device. */
 int spect_plan_create(const spect_geom *g, spect_plan **out);
+/* The same, for callers that trade local accuracy for speed: where the planes'
+ * PSFs vary smoothly, float32 projections, back projections, OSEM steps and
+ * batches of this plan -- without attenuation or with the attenuation field --
+ * blur a few combined images instead of every plane.  A blurred value is then
+ * accurate to about 2^-22 of the largest values within a PSF's reach, not of
+ * itself: the tails of a bright source, and zeros beside it, hold noise of that
+ * size, so data of a large dynamic range (ratios against a projection that is
+ * nearly zero) should not use it; and an infinity or a NaN reaches further than
+ * the PSF, as NaN.  The plan keeps tables that take 0.1 to 0.6 ms of host time
+ * per detector radius, and float32 workspaces are larger. */
+int spect_plan_create_images(const spect_geom *g, spect_plan **out);
 int spect_plan_destroy(spect_plan *p);
 /* Padded side P, pad, PSF half width H used by the kernels and chunk count. */
 int spect_plan_dims(const spect_plan *p, int32_t *padded, int32_t *pad, int32_t *psf_half,

@@ -24,7 +24,7 @@ OUT_STORE, OUT_ADD, OUT_OSEM = 0, 1, 2
 NOALLOC_SCRATCH_BYTES = 128 << 20  # SPECT_NOALLOC_SCRATCH_BYTES
 
 EXPORTED = (
-    "spect_last_error", "spect_version", "spect_plan_create", "spect_plan_destroy",
+    "spect_last_error", "spect_version", "spect_plan_create", "spect_plan_create_images", "spect_plan_destroy",
     "spect_plan_dims", "spect_workspace_bytes", "spect_schedule_info",
     "spect_att_table_bytes", "spect_att_table_build",
     "spect_att_field_bytes", "spect_att_field_build",
@@ -85,6 +85,8 @@ def _declare(lib):
     lib.spect_version.restype = ci
     lib.spect_plan_create.restype = ci
     lib.spect_plan_create.argtypes = [ctypes.POINTER(SpectGeom), ctypes.POINTER(vp)]
+    lib.spect_plan_create_images.restype = ci
+    lib.spect_plan_create_images.argtypes = [ctypes.POINTER(SpectGeom), ctypes.POINTER(vp)]
     lib.spect_plan_destroy.restype = ci
     lib.spect_plan_destroy.argtypes = [vp]
     lib.spect_plan_dims.restype = ci

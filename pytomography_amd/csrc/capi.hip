@@ -311,8 +311,8 @@ int att_rows(const spect_plan *p, const Geo<R> &g, const R *mu, const void *tabl
   return SPECT_OK;
 }
 
-// Whether a float32 call blurs combined images (lowrank.hpp): a PSF that they
-// represent, and the attenuation factors as a field or no attenuation (the
+// Whether a float32 call blurs combined images (lowrank.hpp): a plan that was
+// created for them, a PSF that they represent, and the attenuation factors as a field or no attenuation (the
 // suffix table's march carries a state from plane to plane).
 bool lr_runs(const spect_plan *p, const float *attf, const float *mu) {
   return p->lr.nseg > 0 && (attf || !mu);
@@ -795,7 +795,7 @@ const char *spect_last_error(void) { return g_err.c_str(); }
 
 int spect_version(void) { return SPECT_VERSION; }
 
-int spect_plan_create(const spect_geom *g, spect_plan **out) {
+static int plan_create(const spect_geom *g, bool images, spect_plan **out) {
   if (!g || !out) return fail(SPECT_E_ARG, "null argument");
   *out = nullptr;
   if (g->nx <= 0 || g->ny <= 0 || g->nz <= 0) return fail(SPECT_E_ARG, "object shape must be positive");
@@ -915,7 +915,7 @@ int spect_plan_create(const spect_geom *g, spect_plan **out) {
     if ((rc = upload(&p->taps_z32, z32.data(), z32.size()))) return cleanup(rc);
     auto t32v = tap_tiers<float>(r32.data(), z32.data(), rows, H, kTierEps32);
     if ((rc = upload(&p->tier32, t32v.data(), t32v.size()))) return cleanup(rc);
-    if (!p->has64) {
+    if (images && !p->has64) {
       if ((rc = lowrank_build<float>(p, r32.data(), z32.data()))) return cleanup(rc);
     }
     if (p->has64) {
@@ -925,12 +925,16 @@ int spect_plan_create(const spect_geom *g, spect_plan **out) {
       if ((rc = upload(&p->taps_z64, z64.data(), z64.size()))) return cleanup(rc);
       auto t64v = tap_tiers<double>(r64.data(), z64.data(), rows, H, kTierEps64);
       if ((rc = upload(&p->tier64, t64v.data(), t64v.size()))) return cleanup(rc);
-      if ((rc = lowrank_build<double>(p, r64.data(), z64.data()))) return cleanup(rc);
+      if (images && (rc = lowrank_build<double>(p, r64.data(), z64.data()))) return cleanup(rc);
     }
   }
   *out = p;
   return SPECT_OK;
 }
+
+int spect_plan_create(const spect_geom *g, spect_plan **out) { return plan_create(g, false, out); }
+
+int spect_plan_create_images(const spect_geom *g, spect_plan **out) { return plan_create(g, true, out); }
 
 int spect_plan_destroy(spect_plan *p) {
   if (!p) return SPECT_OK;

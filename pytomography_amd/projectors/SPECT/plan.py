@@ -24,15 +24,17 @@ def _as_ptr(arr: np.ndarray, ctype):
 
 
 class SpectPlan:
-    """Owns one ``spect_plan`` (device tables) for one device."""
+    """Owns one ``spect_plan`` (device tables) for one device; ``images``: a plan
+    whose float32 calls may blur combined images (``spect_plan_create_images``)."""
 
-    def __init__(self, geom_args: dict, device: torch.device):
+    def __init__(self, geom_args: dict, device: torch.device, images: bool = False):
         self.lib = _lib.lib()
         self._keep = geom_args["_keep"]  # host arrays referenced by the geom struct
         g = _lib.SpectGeom(**{k: v for k, v in geom_args.items() if k != "_keep"})
         handle = ctypes.c_void_p()
         with torch.cuda.device(device):
-            _lib.check(self.lib.spect_plan_create(ctypes.byref(g), ctypes.byref(handle)))
+            create = self.lib.spect_plan_create_images if images else self.lib.spect_plan_create
+            _lib.check(create(ctypes.byref(g), ctypes.byref(handle)))
         self.handle = handle
         dims = [ctypes.c_int32() for _ in range(4)]
         _lib.check(self.lib.spect_plan_dims(handle, *[ctypes.byref(d) for d in dims]))

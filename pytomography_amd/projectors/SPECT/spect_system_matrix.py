@@ -59,8 +59,8 @@ class SPECTSystemMatrix(SystemMatrix):
         object_initial_based_on_camera_path: not supported (must be False).
         sensitivity_dtype: dtype of the H^T 1 computation (float64 default).
         chunk_planes: planes per uniform work chunk (0: library default, 16).
-        sched_rounds: for calls that blur every plane (float64, no PSF, derivatives):
-            the forward projection and the back projection's field kernel, without attenuation or with the attenuation field, split
+        sched_rounds: the forward projection and the back projection's field
+            kernel, without attenuation or with the attenuation field, split
             their visited planes evenly over this many rounds of the blocks the
             GPU holds at once; 0 (default) chooses per call: one round when the
             call's pieces of at most 32 planes fit the resident blocks (for the
@@ -73,6 +73,12 @@ class SPECTSystemMatrix(SystemMatrix):
             None: on for float32 when it needs at most ``ATT_FIELD_AUTO_BYTES`` and at
             most ``ATT_FIELD_AUTO_FRACTION`` of the device's memory (e.g. 19 GB at
             256^3 x 180 angles).
+        combined_images: let float32 projections, OSEM steps and batches (without
+            attenuation or with the attenuation field) blur a few combined images
+            that represent the planes' PSFs, where they vary smoothly, instead of
+            every plane.  Faster; a value is then accurate to about 2^-22 of the
+            largest values within a PSF's reach instead of itself
+            (``spect_plan_create_images``).
     """
 
     ATT_FIELD_AUTO_BYTES = 64 << 30
@@ -82,7 +88,7 @@ class SPECTSystemMatrix(SystemMatrix):
                  object_initial_based_on_camera_path: bool = False,
                  sensitivity_dtype: torch.dtype = torch.float64, chunk_planes: int = 0,
                  sched_rounds: int = 0,
-                 attenuation_field: bool | None = None) -> None:
+                 attenuation_field: bool | None = None, combined_images: bool = False) -> None:
         super().__init__(object_meta, proj_meta, obj2obj_transforms, proj2proj_transforms)
         if object_initial_based_on_camera_path:
             raise NotImplementedError("object_initial_based_on_camera_path is not supported")
@@ -99,6 +105,7 @@ class SPECTSystemMatrix(SystemMatrix):
         self.chunk_planes = int(chunk_planes)
         self.sched_rounds = int(sched_rounds)
         self.attenuation_field = attenuation_field
+        self.combined_images = bool(combined_images)
         self._plans: dict = {}
         self._ws: dict = {}
         self._idx32: dict = {}
@@ -134,7 +141,7 @@ class SPECTSystemMatrix(SystemMatrix):
     def _plan(self, device: torch.device) -> SpectPlan:
         key = (device.type, device.index)
         if key not in self._plans:
-            self._plans[key] = SpectPlan(self._geom_args(), device)
+            self._plans[key] = SpectPlan(self._geom_args(), device, self.combined_images)
         return self._plans[key]
 
     def _workspace(self, device, dt: torch.dtype, n: int):
@@ -148,8 +155,7 @@ class SPECTSystemMatrix(SystemMatrix):
 
     def schedule(self, subset_idx: int | None = None, dtype: torch.dtype | None = None) -> dict:
         """The plane schedule that kernels which blur every plane run for this
-        subset's angles (float32 calls with a PSF may blur combined images
-        instead, csrc/lowrank_launch.hpp, and then have none)
+        subset's angles (calls that blur combined images have none)
         (``spect_schedule_info``): ``{"forward": ..., "field": ...}`` with
         "balanced" (pieces of the visited planes over one round of resident
         blocks) or "uniform" (``chunk_planes``-plane chunks); "forward" is the
