@@ -688,9 +688,8 @@ def measure_osem(n: int, na: int, ns: int, att: bool, psf: bool, device, steps: 
     fwd_b, bwd_b, upd_b, ratio_b = algorithmic_bytes(n, a_s, att)
     # Dominant kernel: the forward projection (its projector kernel + the
     # partials' reduce), timed above with HIP events on the stream it is
-    # launched on; which pair runs follows from the PSF and the plane schedule
-    kern = (f"lr_gather_kernel + lr_blur_forward_kernel (spect_forward, {a_s} angles)" if psf
-            else f"fwd_sched_kernel + reduce_sched_kernel (spect_forward, {a_s} angles)"
+    # launched on; which pair runs follows the plane schedule of the call
+    kern = (f"fwd_sched_kernel + reduce_sched_kernel (spect_forward, {a_s} angles)"
             if sm.schedule(0, torch.float32)["forward"] == "balanced"
             else f"fwd_kernel + fwd_reduce_kernel (spect_forward, {a_s} angles)")
     achieved = fwd_b / (fwd_ms * 1e-3) / 1e9
@@ -741,9 +740,8 @@ def measure_osem(n: int, na: int, ns: int, att: bool, psf: bool, device, steps: 
                     "note": ("read as a coalesced stream instead of resampling mu per call; the "
                              "forward's measured HBM bytes include it (traffic vs algorithmic bytes "
                              "in the roofline entry)")}
-    # the plane schedule the timed kernels ran (spect_schedule_info); with a PSF
-    # they blur combined images instead of planes
-    schedule = {"forward": "images", "field": "images"} if psf else sm.schedule(0, torch.float32)
+    # the plane schedule the timed kernels ran (spect_schedule_info)
+    schedule = sm.schedule(0, torch.float32)
     del alg, lk, prob, sm
     torch.cuda.empty_cache()
     return dict(

@@ -125,12 +125,13 @@ int spect_plan_dims(const spect_plan *p, int32_t *padded, int32_t *pad, int32_t 
 size_t spect_workspace_bytes(const spect_plan *p, int dtype, int n);
 
 /* The plane schedule an n-angle call runs with this plan, dtype and the
- * device current now (sched_rounds of spect_geom; a float32 call that blurs
- * combined images, see SPECT_PLANES, runs no such schedule): *forward = 1 when the
+ * device current now (sched_rounds of spect_geom): *forward = 1 when the
  * forward projection (no attenuation, or the attenuation field) runs the
- * balanced schedule, 0 for uniform chunks; *field likewise for the back
- * projection's field kernel.  No counterpart in the reference: a diagnostic of
- * this library's launch choice, for callers that tune or report it. */
+ * balanced schedule, 0 for uniform chunks, 2 when it blurs combined images and
+ * runs no such schedule (spect_plan_create_images; dtype | SPECT_PLANES asks for
+ * the calls that pass that flag); *field likewise for the back projection's
+ * field kernel.  No counterpart in the reference: a diagnostic of this library's
+ * launch choice, for callers that tune or report it. */
 int spect_schedule_info(const spect_plan *p, int dtype, int n, int32_t *forward, int32_t *field);
 
 /* Attenuation table: FP64 suffix sums of mu_rot*dx at every chunk boundary

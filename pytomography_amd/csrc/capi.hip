@@ -975,6 +975,8 @@ size_t spect_workspace_bytes(const spect_plan *p, int dtype, int n) {
 int spect_schedule_info(const spect_plan *p, int dtype, int n, int32_t *forward, int32_t *field) {
   if (!p) return fail(SPECT_E_ARG, "null plan");
   if (!forward || !field) return fail(SPECT_E_ARG, "null output argument");
+  const bool planes = (dtype & SPECT_PLANES) != 0;
+  dtype &= ~SPECT_PLANES;
   if (dtype != SPECT_F32 && dtype != SPECT_F64) return fail(SPECT_E_ARG, "dtype must be F32 or F64");
   if (n <= 0 || n > p->A) return fail(SPECT_E_ARG, "angle count out of range");
   // the same choices as forward_core and backward_impl
@@ -983,6 +985,10 @@ int spect_schedule_info(const spect_plan *p, int dtype, int n, int32_t *forward,
                                      : field_sched_blocks<float>(geo<float>(p));
   const int fb = p->rounds >= 0 ? std::max(1, p->rounds) * per : 0;
   *field = sched_auto_ok(p, n, fb) ? 1 : 0;
+  if (dtype == SPECT_F32 && !planes && p->lr.nseg > 0) {
+    *forward = 2;
+    if (lr_back_pays(geo<float>(p), n)) *field = 2;
+  }
   return SPECT_OK;
 }
 

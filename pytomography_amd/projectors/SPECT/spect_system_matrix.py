@@ -154,11 +154,11 @@ class SPECTSystemMatrix(SystemMatrix):
         return ws, ws.numel()
 
     def schedule(self, subset_idx: int | None = None, dtype: torch.dtype | None = None) -> dict:
-        """The plane schedule that kernels which blur every plane run for this
-        subset's angles (calls that blur combined images have none)
+        """The plane schedule the fused kernels run for this subset's angles
         (``spect_schedule_info``): ``{"forward": ..., "field": ...}`` with
         "balanced" (pieces of the visited planes over one round of resident
-        blocks) or "uniform" (``chunk_planes``-plane chunks); "forward" is the
+        blocks), "uniform" (``chunk_planes``-plane chunks) or "images" (the call
+        blurs combined images: ``combined_images``); "forward" is the
         forward projection without attenuation or with the attenuation field,
         "field" the back projection's field kernel ("none" without attenuation
         and PSF, where the back projection gathers the projection directly)."""
@@ -169,9 +169,11 @@ class SPECTSystemMatrix(SystemMatrix):
         plan = self._plan(device)
         n = int(self._angle_index(subset_idx, device).numel())
         fwd, fld = ctypes.c_int32(), ctypes.c_int32()
-        _lib.check(plan.lib.spect_schedule_info(plan.handle, _lib.dtype_code(dt), n,
+        # calls with the attenuation's suffix table blur no images
+        table = self._att is not None and not self._use_field(device, dt)
+        _lib.check(plan.lib.spect_schedule_info(plan.handle, self._code(dt, None, table), n,
                                                 ctypes.byref(fwd), ctypes.byref(fld)))
-        name = lambda v: "balanced" if v.value else "uniform"
+        name = lambda v: ("uniform", "balanced", "images")[v.value]
         direct = self._att is None and self._psf is None
         return {"forward": name(fwd), "field": "none" if direct else name(fld)}
 

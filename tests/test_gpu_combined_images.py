@@ -1,0 +1,80 @@
+"""System matrices whose caller chose combined images: which calls run them
+(SPECTSystemMatrix.schedule), and those calls against the same ones with every
+plane blurred by its own PSF.
+
+Tolerances: the images represent the planes' kernels to 2^-22 in their L2 norm,
+which over the 41 x 41 values within reach is at most 41 x 0.28 x 2^-22 = 2.7e-6
+of the largest value (0.28: the norm of a kernel one pixel wide), and either side
+sums up to 400 terms in float32, sqrt(400) 2^-23 = 2.4e-6: 1e-5 of the largest
+value, and 5e-6 in relative L2."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from pytomography_amd import _lib
+from tests.helpers import problem_arrays, product_system_matrix, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TOL, TOL_MAX = 5e-6, 1e-5
+
+
+def images_matrix(pa, **kw):
+    sm = product_system_matrix(pa, **kw)
+    assert not sm._plans
+    sm.combined_images = True  # as the constructor's argument, before the first plan
+    return sm
+
+
+# problem, forward and back projection on images (the latter with enough samples
+# of the extended detector: lr_back_pays)
+CASES = {
+    "few_samples": (dict(n=32, n_angles=20, att=True), True, False),
+    "many_samples": (dict(n=32, n_angles=32, att=True), True, True),
+    "aligned_slices": (dict(n=64, n_angles=9, att=True), True, True),
+    "ragged_slices": (dict(n=47, n_angles=24, nz=35, att=True), True, True),
+    "one_slice": (dict(n=40, n_angles=7, nz=1), True, False),
+    "no_attenuation": (dict(n=48, n_angles=20), True, True),
+    "table": (dict(n=48, n_angles=20, att=True, field=False), False, False),
+    "contour": (dict(n=72, n_angles=10, att=True, contour=True), True, True),
+    "wide": (dict(n=66, n_angles=12, att=True, radius=75.0), True, True),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_calls_that_run_images(name):
+    c, forward, back = CASES[name]
+    c = dict(c)
+    field, contour, radius = c.pop("field", None), c.pop("contour", False), c.pop("radius", None)
+    pa = problem_arrays(c.pop("n"), c.pop("n_angles"), seed=4, psf=True, **c)
+    if radius:
+        pa["radii"] = np.full(len(pa["radii"]), radius)
+    if contour:
+        pa["radii"] = 22.0 + 3.0 * np.cos(2 * np.deg2rad(pa["angles"]))
+    sm = images_matrix(pa, attenuation_field=field)
+    plain = product_system_matrix(pa, attenuation_field=field).schedule()
+    want = {"forward": "images" if forward else plain["forward"],
+            "field": "images" if back else plain["field"]}
+    assert "images" not in plain.values() and sm.schedule() == want
+    assert sm.schedule(dtype=torch.float64)["forward"] != "images"
+    f = torch.from_numpy(pa["f"]).cuda()
+    rng = np.random.default_rng(2)
+    p = torch.from_numpy((0.5 + rng.random((len(pa["radii"]), pa["n"], pa["nz"]))).astype(np.float32)).cuda()
+    sign = torch.from_numpy(rng.choice([-1.0, 1.0], p.shape).astype(np.float32)).cuda()
+
+    def compare(what, a, b, scale, ran):
+        err, most = rel_l2(a, b), float((a - b).abs().max()) / scale
+        print(f"[{name}] {what}: rel-L2 {err:.1e}, largest {most:.1e}")
+        assert err <= TOL and most <= TOL_MAX
+        assert ran or torch.equal(a, b)
+
+    for x in (f, -f):
+        b = sm._project(x, None, "spect_forward", planes=True)
+        compare("forward", sm.forward(x), b, float(b.abs().max()), forward)
+    for y in (p, p * sign):
+        for mode in (_lib.BP_REFERENCE, _lib.BP_ADJOINT):
+            top = float(sm._backward(y.abs(), None, mode, planes=True).max())
+            compare(f"back projection {mode}", sm._backward(y, None, mode),
+                    sm._backward(y, None, mode, planes=True), top, back)
