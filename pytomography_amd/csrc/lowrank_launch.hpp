@@ -79,8 +79,9 @@ inline int lr_zblocks(int Nz) { return (Nz + 63) / 64; }
 // with attenuation: 64^3 x 4 angles 27.3 / 27.5 us, x 8 35.4 / 33.3, x 16
 // 46.6 / 39.7; 80^3 x 4 31.1 / 34.9, x 8 42.9 / 39.2; 128^3 x 2 33.3 / 38.3,
 // x 4 49.6 / 43.9, x 16 144 / 108.  (The forward's two launches replace two:
-// 64^3 x 2 27.8 / 19.4, 128^3 x 16 105 / 85.)
-constexpr long long kLrBackSamples = 39000;
+// 64^3 x 2 27.8 / 19.4, 128^3 x 16 105 / 85.)  The line lies between 128^3 x 2
+// (39936 samples of the extended detector) and 64^3 x 8 (43008).
+constexpr long long kLrBackSamples = 41000;
 inline bool lr_back_pays(const Geo<float> &g, int n) {
   return (long long)n * (g.je1 - g.je0) * g.Nz >= kLrBackSamples;
 }
