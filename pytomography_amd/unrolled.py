@@ -98,12 +98,13 @@ class UnrolledBSREM:
 
     # The iterations and their derivative blur every plane with its own PSF, as
     # backward_transpose does: the operators that are differentiated are the
-    # ones that are applied.  (A system matrix with projections of its own, or
-    # on the per-angle path, is called as it is.)
+    # ones that are applied.  (A system matrix with projections of its own -- a
+    # subclass's, or a wrapper put on the object or the class -- or on the
+    # per-angle path is called as it is.)
     def _own(self, name) -> bool:
-        from pytomography_amd.projectors.SPECT import SPECTSystemMatrix
-        return (getattr(type(self.sm), name, None) is not getattr(SPECTSystemMatrix, name)
-                or not self.sm.fused)
+        from pytomography_amd.projectors.SPECT.spect_system_matrix import FUSED_PROJECTIONS
+        called = getattr(getattr(self.sm, name), "__func__", None)
+        return called is not FUSED_PROJECTIONS[name] or not self.sm.fused
 
     def _forward(self, x, k):
         if self._own("forward"):
