@@ -8,7 +8,9 @@ runs OSEM for many problems of uneven size and angle count at once: each
 sub-iteration launches every kernel once for all problems that share a PSF
 width and z extent (``spect_batch_*`` in include/spect_hip.h), and the whole
 schedule can be captured into one hipGraph and replayed.  Each problem's
-arithmetic is that of ``OSEM`` on its own ``SPECTSystemMatrix``.
+arithmetic is that of ``OSEM`` on its own ``SPECTSystemMatrix``, except that the
+planes' partial sums are those of uniform chunks, and that problems with
+``combined_images`` choose how they back-project by the size of the whole launch.
 """
 from __future__ import annotations
 

@@ -485,7 +485,9 @@ struct spect_batch {
 
 namespace {
 
-// Whether a batched problem blurs combined images, as its single calls do.
+// Whether a batched problem blurs combined images.  Its single calls' forward
+// projections do as well; the back projection follows the samples of the whole
+// launch, so members that are small by themselves may run images together.
 template <typename R> bool batch_images(const spect_batch_problem &pb) {
   if constexpr (sizeof(R) == 4) return pb.plan->lr.nseg > 0 && (pb.att_field || !pb.mu);
   else return false;
@@ -522,7 +524,7 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
   auto put = [&](const void *src, size_t bytes) {
     const size_t off = (host.size() + 255) & ~size_t(255);
     host.resize(off + bytes);
-    std::memcpy(host.data() + off, src, bytes);
+    if (bytes) std::memcpy(host.data() + off, src, bytes);
     return off;
   };
   for (size_t k = 0; k < keys.size(); ++k) {
@@ -558,11 +560,13 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
         const R *attf = pb.att_field ? reinterpret_cast<const R *>(pb.att_table) : nullptr;
         const int32_t *idx = pb.angle_idx[sub];
         R *f = reinterpret_cast<R *>(pb.f);
-        fj.push_back(FwdJob<R>{g, tb, f, mu, att, 1, attf, idx, cnt, part});
-        rj.push_back(ReduceJob<R>{g, part, cnt, nullptr, reinterpret_cast<const R *>(pb.g[sub]),
-                                  pb.s ? reinterpret_cast<const R *>(pb.s[sub]) : nullptr,
-                                  pb.pred ? reinterpret_cast<R *>(pb.pred[sub]) : nullptr, ratio,
-                                  R(delta)});
+        const ReduceJob<R> red{g, part, cnt, nullptr, reinterpret_cast<const R *>(pb.g[sub]),
+                               pb.s ? reinterpret_cast<const R *>(pb.s[sub]) : nullptr,
+                               pb.pred ? reinterpret_cast<R *>(pb.pred[sub]) : nullptr, ratio, R(delta)};
+        if (!G.images) {
+          fj.push_back(FwdJob<R>{g, tb, f, mu, att, 1, attf, idx, cnt, part});
+          rj.push_back(red);
+        }
         lj.push_back(FieldJob<R>{g, tb, ratio, mu, att, 1, attf, idx, cnt, W, nullptr, nullptr, nullptr});
         gj.push_back(GatherJob<R>{g, tb, W, idx, cnt, SPECT_OUT_OSEM, f, f,
                                   reinterpret_cast<const R *>(pb.norm[sub]), R(delta),
@@ -571,7 +575,7 @@ int batch_build(spect_batch *b, const spect_batch_problem *probs, int n, double 
           if (G.images) {
             const LrGatherJob J = lr_gather_job(g, tb, p->lr, f, attf, idx, cnt, ws + l.part_off);
             lb.gather.push_back(J);
-            lb.blur.push_back(lr_blur_job(J, nullptr, rj.back().gm, rj.back().s, rj.back().pred, ratio, R(delta)));
+            lb.blur.push_back(lr_blur_job(J, nullptr, red.gm, red.s, red.pred, ratio, R(delta)));
             lb.back.push_back(lr_back_job(g, tb, p->lr, ratio, attf, idx, cnt, W, ws + l.q_off));
           }
         }
@@ -620,8 +624,9 @@ int batch_launch_group(spect_batch *b, const spect_batch::Group &G, int n_iters,
         HIP_TRY(launch_lr_batch_forward(G.lr[sub], reinterpret_cast<const LrGatherJob *>(base + G.lr_off[0][sub]),
                                         reinterpret_cast<const LrBlurJob *>(base + G.lr_off[1][sub]), starts(0),
                                         starts(1), st));
-        HIP_TRY(launch_lr_batch_field(G.lr[sub], reinterpret_cast<const LrBackJob *>(base + G.lr_off[2][sub]),
-                                      starts(2), starts(3), st));
+        if (G.lr[sub].back_pays)
+          HIP_TRY(launch_lr_batch_field(G.lr[sub], reinterpret_cast<const LrBackJob *>(base + G.lr_off[2][sub]),
+                                        starts(2), starts(3), st));
       } else {
         HIP_TRY(launch_forward_batch<R>(reinterpret_cast<const FwdJob<R> *>(base + G.fwd_off[sub]),
                                         reinterpret_cast<const int *>(base + G.starts_off[0][sub]),
@@ -629,10 +634,11 @@ int batch_launch_group(spect_batch *b, const spect_batch::Group &G, int n_iters,
         HIP_TRY(launch_reduce_batch<R>(reinterpret_cast<const ReduceJob<R> *>(base + G.red_off[sub]),
                                        reinterpret_cast<const int *>(base + G.starts_off[1][sub]),
                                        G.nprob, G.blocks[1][sub], st));
+      }
+      if (!G.images || !G.lr[sub].back_pays)
         HIP_TRY(launch_field_batch<R>(reinterpret_cast<const FieldJob<R> *>(base + G.fld_off[sub]),
                                       reinterpret_cast<const int *>(base + G.starts_off[2][sub]),
                                       G.nprob, G.blocks[2][sub], G.H, G.Nz, G.maxL, G.af, st));
-      }
       HIP_TRY(launch_gather_batch<R>(reinterpret_cast<const GatherJob<R> *>(base + G.gat_off[sub]),
                                      reinterpret_cast<const int *>(base + G.starts_off[3][sub]),
                                      G.nprob, G.blocks[3][sub], SPECT_BP_REFERENCE, st));

@@ -255,7 +255,7 @@ hipError_t launch_lr_field(LrBackJob J, size_t scratch_bytes, hipStream_t st) {
 }
 
 bool lr_batch_finish(LrBatch &b) {
-  long long two = 0, four = 0, back = 0;
+  long long two = 0, four = 0, back = 0, samples = 0;
   size_t field = 0;
   int nimg = 0;
   for (size_t i = 0; i < b.gather.size(); ++i) {
@@ -264,11 +264,13 @@ bool lr_batch_finish(LrBatch &b) {
     four += blur_items(b.blur[i], 4);
     b.back[i].jranges = lr_back_ranges(g, kLrBackTiles);
     back += back_items(b.back[i]);
+    samples += lr_back_samples(g, b.back[i].n);
     nimg = std::max(nimg, b.gather[i].lr.nimg);
     field += (size_t)g.A * g.P * (g.je1 - g.je0) * g.Nz * sizeof(float);
   }
   b.row_tiles = forward_tiles(two, four);
   b.back_tiles = backward_tiles(back);
+  b.back_pays = samples >= kLrBackSamples;
   b.waves = blur_waves(nimg);
   b.H = b.gather[0].g.H;
   b.Nz = b.gather[0].g.Nz;

@@ -82,9 +82,8 @@ inline int lr_zblocks(int Nz) { return (Nz + 63) / 64; }
 // 64^3 x 2 27.8 / 19.4, 128^3 x 16 105 / 85.)  The line lies between 128^3 x 2
 // (39936 samples of the extended detector) and 64^3 x 8 (43008).
 constexpr long long kLrBackSamples = 41000;
-inline bool lr_back_pays(const Geo<float> &g, int n) {
-  return (long long)n * (g.je1 - g.je0) * g.Nz >= kLrBackSamples;
-}
+inline long long lr_back_samples(const Geo<float> &g, int n) { return (long long)n * (g.je1 - g.je0) * g.Nz; }
+inline bool lr_back_pays(const Geo<float> &g, int n) { return lr_back_samples(g, n) >= kLrBackSamples; }
 
 // Columns and z of a wave in the first forward pass (lr_gather_body).
 constexpr int kLrGatherCols = 2;
@@ -172,6 +171,8 @@ hipError_t launch_lr_field(LrBackJob J, size_t scratch_bytes, hipStream_t st);
 // The four passes of several calls with one Nz and one class of half widths
 // (H <= 16 or not), all with attenuation factors or all without, in one launch
 // each.
+// back_pays: whether the launch's samples make the back projection on images
+// the faster one (lr_back_pays, of all calls together).
 struct LrBatch {
   std::vector<LrGatherJob> gather;
   std::vector<LrBlurJob> blur;
@@ -179,6 +180,7 @@ struct LrBatch {
   std::vector<int> starts[4];  // first block of each call: gather, blur, back blur, field
   int blocks[4];
   int row_tiles, back_tiles, waves, factor_mode, H, Nz;
+  bool back_pays;
 };
 // Fills everything that follows from gather, blur and back.
 bool lr_batch_finish(LrBatch &b);
