@@ -155,13 +155,20 @@ def _osem_step_seconds(sm, n: int, n_subsets: int, device, reps: int) -> float:
     return (time.perf_counter() - t0) / reps
 
 
-def _tune(key: str, device, candidates, seconds):
+def _tune(key: str, device, candidates, seconds, untimed=None):
+    """The fastest candidate, from the cache when it is there.  ``untimed()``: the
+    answer for calls that no candidate reaches, or None."""
     device = device or pytomography_amd.device
     cache = _load_cache()
-    ck = f"{torch.cuda.get_device_name(device)}|{key}"
+    # what is timed blurs every plane, in this dtype
+    dt = "float64" if pytomography_amd.dtype == torch.float64 else "float32"
+    ck = f"{torch.cuda.get_device_name(device)}|{dt}|planes|{key}"
     if ck in cache:
         v = cache[ck]
         return tuple(v) if isinstance(v, list) else int(v)
+    answer = untimed() if untimed is not None else None
+    if answer is not None:
+        return answer
     best, best_t = None, float("inf")
     for cand in candidates:
         t = seconds(cand, device)
@@ -170,6 +177,18 @@ def _tune(key: str, device, candidates, seconds):
     cache[ck] = list(best) if isinstance(best, tuple) else best
     _store_cache()
     return best
+
+
+def _library_choice(sm, n_subsets: int, default, candidates):
+    """The library's own value where the whole sub-iteration of subset 0 blurs
+    combined images: the tuned values reach none of its kernels, and timing noise
+    would choose among them."""
+    if not sm.combined_images:
+        return None
+    sm.set_n_subsets(n_subsets)
+    if sm.schedule(0)["field"] != "images":
+        return None
+    return default if default in candidates else candidates[0]
 
 
 def _batch_iteration_seconds(sm, n: int, n_angles: int, n_subsets: int, device, reps: int) -> float:
@@ -195,10 +214,14 @@ def autotune_chunk_planes(make_system_matrix, n: int, n_angles: int, n_subsets: 
     batch on the device.
 
     ``make_system_matrix(chunk_planes)`` builds a system matrix of the class.
-    Results are cached per device name and key."""
+    Results are cached per device name, dtype and key.  For batches that blur
+    combined images, which have no chunks, the answer is the library's length,
+    untimed and not cached."""
+    candidates = tuple(candidates)
     return _tune("batch|" + key, device, candidates,
                  lambda c, dev: _batch_iteration_seconds(make_system_matrix(c), n, n_angles,
-                                                         n_subsets, dev, reps))
+                                                         n_subsets, dev, reps),
+                 lambda: _library_choice(make_system_matrix(candidates[0]), n_subsets, 16, candidates))
 
 
 # (chunk_planes, sched_rounds): the library's per-call choice, the balanced
@@ -216,6 +239,11 @@ def autotune_schedule(make_system_matrix, n: int, n_angles: int, n_subsets: int,
     uniform chunks of a plane count.
 
     ``make_system_matrix(chunk_planes, sched_rounds)`` builds a system matrix
-    of the class.  Results are cached per device name and key."""
+    of the class.  Results are cached per device name, dtype and key.  Where the
+    sub-iteration blurs combined images, which have no schedule, the answer is the
+    library's per-call choice, untimed and not cached."""
+    candidates = tuple(candidates)
     return _tune("sched|" + key, device, candidates,
-                 lambda c, dev: _osem_step_seconds(make_system_matrix(*c), n, n_subsets, dev, reps))
+                 lambda c, dev: _osem_step_seconds(make_system_matrix(*c), n, n_subsets, dev, reps),
+                 lambda: _library_choice(make_system_matrix(*candidates[0]), n_subsets, (0, 0),
+                                         candidates))
