@@ -25,6 +25,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <exception>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -214,19 +216,31 @@ bool lowrank_tables(const T *taps_y, const T *taps_z, int n_radii, int P, int H,
   const int K = 2 * H + 1, units = (P + kLrUnit - 1) / kLrUnit;
   for (size_t k = 0; k < (size_t)n_radii * P * K; ++k)
     if (!(taps_y[k] >= T(0)) || !(taps_z[k] >= T(0))) return false;
-  // a body-contour orbit has a radius per angle, 0.1 to 0.4 ms each: a thread
-  // per 16 radii
+  // a body-contour orbit has a radius per angle, 0.1 to 0.6 ms each: a thread
+  // per 16 radii, this one for those that the system does not give.  Nothing may
+  // leave a thread, nor this function with threads running: the entry is C.
   std::vector<LrRadius> fits(n_radii);
   std::vector<char> ok(n_radii, 0);
   const int nt = std::max(1, std::min(8, n_radii / 16));
-  auto work = [&](int first) {
-    for (int r = first; r < n_radii; r += nt)
-      ok[r] = lowrank_fit<T>(taps_y + (size_t)r * P * K, taps_z + (size_t)r * P * K, P, H, fits[r]) ? 1 : 0;
+  auto work = [&](int first) noexcept {
+    for (int r = first; r < n_radii; r += nt) {
+      try {
+        ok[r] = lowrank_fit<T>(taps_y + (size_t)r * P * K, taps_z + (size_t)r * P * K, P, H, fits[r]) ? 1 : 0;
+      } catch (const std::exception &) {  // out of memory: blur planes
+      }
+    }
   };
-  std::vector<std::thread> threads;
-  for (int k = 1; k < nt; ++k) threads.emplace_back(work, k);
+  std::vector<std::thread> threads(nt);
+  for (int k = 1; k < nt; ++k) {
+    try {
+      threads[k] = std::thread(work, k);
+    } catch (const std::system_error &) {
+      work(k);
+    }
+  }
   work(0);
-  for (auto &th : threads) th.join();
+  for (auto &th : threads)
+    if (th.joinable()) th.join();
   t = LrHostTables{};
   for (int r = 0; r < n_radii; ++r) {
     if (!ok[r]) return false;
