@@ -266,7 +266,8 @@ class SPECTSystemMatrix(SystemMatrix):
         """H_m^T 1 (spect_system_matrix.py:106-118), computed in
         ``sensitivity_dtype`` on the GPU and returned in the working dtype."""
         device = pytomography_amd.device
-        if self.fused and self._psf is not None and self.sensitivity_dtype == torch.float64:
+        if (self.fused and self._psf is not None and self.sensitivity_dtype == torch.float64
+                and torch.device(device).type == "cuda"):
             return self._sensitivity(subset_idx).to(pytomography_amd.dtype)
         n = self.proj_meta.num_projections if subset_idx is None else len(self.subset_indices_array[subset_idx])
         ones = torch.ones((n, *self.proj_meta.shape[1:]), dtype=self.sensitivity_dtype, device=device)
