@@ -1,11 +1,12 @@
 // lowrank.hpp -- the PSF of all planes as combinations of a few planes' PSFs
 // (host code).
 //
-// The taps of plane i are a Gaussian (or any profile) whose width varies
-// smoothly with the distance to the detector, so the planes' 2-D kernels
-// k_i = y taps (x) z taps span, numerically, far fewer dimensions than there
-// are planes: over a range of planes whose widths differ by at most a factor
-// of two, about ten of them reproduce every other one to 2^-22 of its norm
+// For plans whose caller chose it (spect_plan_create_images).  The taps of plane
+// i are a Gaussian (or any profile) whose width varies smoothly with the distance
+// to the detector, so the planes' 2-D kernels k_i = y taps (x) z taps span,
+// numerically, far fewer dimensions than there are planes: over a range of planes
+// whose widths differ by at most a factor of two, about ten of them reproduce
+// every other one to 2^-22 of its norm
 // (128^3 at 4.8 mm, sigma = 0.03 d + 0.1 cm: 29 kernels for 182 planes).  With
 //   k_i = sum_r c[i][r] k_(node r)
 // the ray sum of blurred planes is the sum of a few blurred images,
@@ -15,10 +16,13 @@
 // Planes are taken in units of 16 (one MFMA tile of planes).  Consecutive
 // units form a group while their widths (plus kLrWidthOffset: narrow kernels
 // reach few pixels whatever their ratio) stay within kLrRatio of each other: a
-// node is then never much wider than the planes it stands for, so the rounding
-// of the combination stays below the planes' own tails (one basis for all
+// node is then never much wider than the planes it stands for (one basis for all
 // planes would need 20 images instead of 29, but puts 2^-24 of the widest
-// kernel under the narrowest).  Consecutive groups whose nodes fill at most
+// kernel under the narrowest).  The planes' tails are not kept: where a plane's
+// own tap is smaller, up to 6e-8 of its peak remains of the combination, and tap
+// products above 1e-4 of the peak are off by up to 1.6e-3 of themselves.  Keeping
+// every tap within 1e-6 of itself takes a width ratio of 1.2 and 90 images at
+// 128^3, whose blurs cost as much as the planes'.  Consecutive groups whose nodes fill at most
 // kLrRows rows share a segment (one MFMA tile of images).
 #pragma once
 
